@@ -126,6 +126,10 @@ def load() -> ctypes.CDLL:
         lib.mk_prefill_workspace_bytes.restype = c_size_t
         lib.mk_sample.argtypes = [POINTER(MkSampleArgs)]
         lib.mk_sample.restype = c_int
+        lib.mk_sample_scratch_bytes.argtypes = [c_int32, c_int32]
+        lib.mk_sample_scratch_bytes.restype = c_size_t
+        lib.mk_sample_with_scratch.argtypes = [POINTER(MkSampleArgs), c_void_p, c_size_t]
+        lib.mk_sample_with_scratch.restype = c_int
         lib.mk_sample_last_error.restype = c_char_p
         if lib.mk_abi_version() != ABI_VERSION:
             raise RuntimeError(f"{LIB_PATH} has ABI version {lib.mk_abi_version()}, this module {ABI_VERSION}: "
@@ -380,7 +384,7 @@ def prepare_sampling_params(batch_size: int, top_k, top_p, temperature, device="
 
 def sample(logits: torch.Tensor, params: torch.Tensor, tokens_out: torch.Tensor, *, seed: int = 0,
            counter: Optional[torch.Tensor] = None, uniforms_out: Optional[torch.Tensor] = None) -> None:
-    """``mk_sample`` on the current stream: next tokens from fp32 logits [B, V]
+    """``mk_sample_with_scratch`` on the current stream: next tokens from fp32 logits [B, V]
     with per-row (top_k, top_p, temperature); ``counter`` [B] int32 (e.g. the
     positions) feeds the Philox counter."""
     if logits.dtype != torch.float32 or logits.dim() != 2 or logits.stride(1) != 1:
@@ -392,7 +396,12 @@ def sample(logits: torch.Tensor, params: torch.Tensor, tokens_out: torch.Tensor,
         raise ValueError("tokens_out must be int32 with at least B elements")
     a = MkSampleArgs(logits.data_ptr(), B, V, logits.stride(0), params.data_ptr(), seed & 0xFFFFFFFFFFFFFFFF,
                      _ptr(counter), tokens_out.data_ptr(), _ptr(uniforms_out), current_stream_ptr())
-    rc = load().mk_sample(ctypes.byref(a))
+    # scratch from torch's allocator: its own for every call, and ordered by the current stream
+    # (under a capture it comes from the graph's pool)
+    lib = load()
+    n = lib.mk_sample_scratch_bytes(B, V)
+    scratch = torch.empty(n, dtype=torch.uint8, device=logits.device) if n else None
+    rc = lib.mk_sample_with_scratch(ctypes.byref(a), _ptr(scratch), n)
     if rc != MK_OK:
         raise MkError(rc, load().mk_sample_last_error().decode(errors="replace"))
 

@@ -128,3 +128,75 @@ def test_generate_with_sampling():
         assert int(out1[t]) == ref, (t, int(out1[t]), ref)
     greedy = m.generate(ids, 8)
     say(f"[sample] generate: sampled {out1[:8].tolist()} greedy {greedy.tolist()}")
+
+
+def _edge_row(kind, V, g):
+    """Rows that steer the sampler's candidate search: see the cases below."""
+    x = torch.randn(V, generator=g) * 2
+    if kind == "sorted":          # the best logits side by side: too many in the candidates' groups
+        x = x.sort(descending=True).values
+    elif kind == "masked":        # a grammar mask: few tokens allowed, the rest tie at -inf
+        keep = torch.randperm(V, generator=g)[:max(1, min(40, V // 2))]
+        y = torch.full((V,), float("-inf"))
+        y[keep] = x[keep]
+        x = y
+    elif kind == "lowest":        # masked with the type's lowest value instead
+        x[torch.randperm(V, generator=g)[:V - max(1, V // 100)]] = torch.finfo(torch.float32).min
+    elif kind == "steps":         # few distinct values: ties at every threshold
+        x = x.round() + 0.0     # (no -0)
+    elif kind == "equal":
+        x = torch.full((V,), 1.5)
+    elif kind == "nan":           # never drawn while enough numbers are there
+        x[torch.randperm(V, generator=g)[:V // 7]] = float("nan")
+    return x.float()
+
+
+@pytest.mark.parametrize("pad", [0, 3])
+@pytest.mark.parametrize("V", [1, 2, 63, 1025, 4095, 4096, 4097, 4500, 32768, 32769, 128255, 131073])
+def test_sample_edges(V, pad):
+    """Vocabularies at the edges of the candidate search (whole rows sorted up
+    to 4096, then groups of 4, 8, 16, 32 logits), row strides that break the
+    16-byte alignment, and rows that tie, cluster or mask: the same tokens with
+    and without scratch, and the oracle's, or a token of its CDF bracket
+    widened by 1e-5 (fp32 sums). Where more than 2048 tokens tie at the top-k
+    threshold only the tokens above it are certain: the draw is one of the
+    tokens at or above it."""
+    need_gpu()
+    import ctypes
+    import mk_lib
+    from oracle.sampling_ref import cdf_bracket, sample
+    g = torch.Generator().manual_seed(V + pad)
+    rows = [(kind, k, tp) for kind in ("normal", "sorted", "masked", "lowest", "steps", "equal", "nan")
+            for k, tp in ((1, 1.0), (2, 1.0), (50, 0.9), (700, 0.95), (0, 1.0))]
+    B = len(rows)
+    store = torch.zeros(B, V + pad)
+    for b, (kind, _, _) in enumerate(rows):
+        store[b, :V] = _edge_row(kind, V, g)
+    dev = store.cuda()
+    logits = dev[:, :V]
+    params = torch.tensor([(k, tp, 0.8) for _, k, tp in rows], dtype=torch.float32).cuda()
+    counter = torch.arange(B, dtype=torch.int32).cuda()
+    tok, u = run(logits, params, 21, counter)
+    plain = torch.full((B,), -7, dtype=torch.int32, device="cuda")
+    a = mk_lib.MkSampleArgs(logits.data_ptr(), B, V, logits.stride(0), params.data_ptr(), 21, counter.data_ptr(),
+                            plain.data_ptr(), None, mk_lib.current_stream_ptr())
+    assert mk_lib.load().mk_sample(ctypes.byref(a)) == 0
+    torch.cuda.synchronize()
+    plain = plain.cpu().numpy()
+    for b, (kind, k, tp) in enumerate(rows):
+        x = store[b, :V].numpy()
+        y = np.where(np.isnan(x), -np.inf, x)          # the sampler's order puts NaN below every number
+        if kind == "nan" and 0 < k <= 1024 and k > np.isfinite(x).sum() or kind == "nan" and k == 0 and np.isfinite(x).sum() < 1024:
+            continue                                   # NaN among the kept: no distribution to check
+        kk = min(k if 0 < k <= 1024 else 1024, V)
+        at_least = int((y >= np.sort(y)[::-1][kk - 1]).sum())
+        if k != 1 and at_least > 2048:
+            thr = np.sort(y)[::-1][kk - 1]
+            assert y[tok[b]] >= thr and y[plain[b]] >= thr, (kind, k, int(tok[b]), int(plain[b]))
+            continue
+        assert tok[b] == plain[b], (kind, k, int(tok[b]), int(plain[b]))
+        ref, ref_u = sample(y, k, tp, 0.8, 21, b, b)
+        if tok[b] != ref:
+            assert k != 1, (kind, int(tok[b]), ref)
+            lo, hi = cdf_bracket(y, k, tp, 0.8, int(tok[b]))
+            assert lo - 1e-5 <= ref_u < hi + 1e-5, (kind, k, int(tok[b]), ref, lo, hi, ref_u)
