@@ -20,17 +20,14 @@
 // attention.py / mlp.py). The last layer runs only its QKV GEMM (its K/V
 // rows are the prefill's output) unless the caller asks for the hidden state.
 //
-// GEMMs: bf16 v_mfma_f32_16x16x32_bf16 with fp32 accumulation, a 128x128
-// output tile per 256-thread workgroup, 64x64 per wave (16 MFMA tiles). The
+// GEMMs (pf_gemm): bf16 v_mfma_f32_16x16x32_bf16 with fp32 accumulation. The
 // activations are kept in A-tile order (the producing kernel writes them so)
-// and the weights are the MFMA-tiled copies, so each k-step's operands of the
-// tile are 16 blocks of 1 KiB, which the four waves copy from memory straight
-// into LDS (one contiguous 1 KiB copy each, four per wave) three k-steps ahead
-// of their use; each wave reads its 4 A and 4 B operands of a k-step from LDS
-// (a block per instruction, conflict-free) and runs 16 MFMAs. The O and down
-// projections of short prompts (few row tiles) split K across workgroups into
-// fp32 partials that pf_reduce_norm sums in a fixed order; so does the QKV
-// projection, whose tail (pf_qkv_finish) then applies RoPE and scatters.
+// and the weights are the MFMA-tiled copies, so each k-step's operands of an
+// output tile are blocks of 1 KiB that go from memory straight into LDS. The
+// tile (64x64 to 256x256) and, for short prompts, a split of K into fp32
+// partials are chosen per projection by estimated time (gemm_plan); the
+// partials are summed in a fixed order by pf_reduce_norm (O and down) and
+// pf_qkv_finish (QKV, with RoPE and the scatter).
 //
 // Attention: per (kv head, block of 16 tokens) one workgroup; S^T = K Q^T on
 // the matrix cores (keys on M, the 16 tokens x 4 q heads on N), an online
@@ -38,6 +35,7 @@
 // p rounded to bf16 as the reference rounds it (relative to the running
 // maximum). K and V tiles of 32 keys go through LDS (V transposed there).
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 #include <string.h>
 
@@ -49,17 +47,16 @@ namespace {
 
 using namespace mk;
 
-constexpr int PF_TM = 128, PF_TN = 128;   // GEMM output tile per workgroup
 constexpr int PF_TB = 16;                 // tokens per attention workgroup
 
 enum : int { EPI_QKV = 0, EPI_RES = 1, EPI_SWIGLU = 2, EPI_PART = 3 };
-constexpr int GEMM_NS = 4;   // k-steps of operands in flight per wave (a ring of register stages)
 
 struct GemmArgs {
   const uint16_t* a;     // activations, A-tile order [M16][K]
   const uint16_t* b;     // weights [N][K]: MFMA tile order (tiled) or row-major
   int tiled;
   int M, N, K;
+  int mt;                // row tiles
   int splits;            // EPI_PART: the K range is cut into `splits` parts (blockIdx.y)
   const uint16_t* res;   // EPI_RES: residual, row-major [M][N]
   uint16_t* out;         // EPI_RES: row-major [M][N]; EPI_SWIGLU: A-tile order [M16][N/2]; EPI_QKV: q [M][2048]
@@ -72,220 +69,291 @@ struct GemmArgs {
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
-// One k-step of a workgroup's 128x128 tile in LDS: the 8 A blocks (16 rows x
-// 32 columns each, 1 KiB, MFMA A-operand lane order) and the 8 B blocks.
-struct GemmStage {
-  u32x4 a[8][64];
-  u32x4 b[8][64];
-};
-struct GemmLds {
-  GemmStage st[GEMM_NS];
-};
-// The epilogue's side input in LDS: PF_TM rows of 128 bf16, padded to 136
-// (a 272-byte row stride spreads the rows of one read over the banks).
-constexpr int SIDE_LD = 136;
-static_assert(PF_TM * SIDE_LD * 2 <= (int)sizeof(GemmLds), "side input over the operand stages");
+// This wave's copies up to the last N have landed and its LDS reads up to the
+// last R have returned, and so have every wave's.
+template <int N, int R>
+__device__ __forceinline__ void wait_copies() {
+  static_assert(N < 64 && R < 16, "wait counts");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(%1)\n\ts_barrier" ::"n"(N), "n"(R) : "memory");
+}
 
-template <int EPI>
-__global__ void __launch_bounds__(NT) pf_gemm(GemmArgs g) {
-  __shared__ GemmLds L;
-  const int wave = __builtin_amdgcn_readfirstlane(wave_id()), lane = lane_id();   // (uniform: LDS copy bases)
-  const int nbn = g.N / PF_TN;
-  const int tm = blockIdx.x / nbn, tn = blockIdx.x % nbn;
-  const int m16 = (g.M + 15) / 16;
+// C = A B^T, one (16 MI WM) x (16 NI WN) output tile per workgroup of WM x WN
+// waves, 16 MI x 16 NI of it per wave.
+//
+// What bounds it: a k-step of 32 columns costs the tile's MFMAs (16 cycles
+// each), the copies of its operands into the CU (64 B/cycle) and their traffic
+// through LDS (128 B/cycle, written once and read by every wave that uses them).
+// A 128x128 tile of 64x64 per wave (the only one before) takes 256 cycles of
+// each at one wave per SIMD and got 770-850 TFLOP/s; 256x256 on eight waves of
+// 128x64 halves the copies per MFMA and puts two waves on a SIMD, so that one
+// multiplies while the other waits: 16384 x 2048 weights at 3000 tokens 208 ->
+// 147 us (1370 TFLOP/s). Smaller tiles serve the shapes that would leave the
+// device idle (gemm_plan).
+//
+// Operands are 1 KiB blocks (16 rows x 32 columns) copied from memory straight
+// into a ring of NS k-steps in LDS, NS - 1 ahead; each wave reads the next
+// k-step's operands into registers while it multiplies the current one
+// (interleaved one read per few MFMAs; without that 1180 instead of 1370).
+// Copies past the operands (k-steps >= ke, rows past the matrix) write zeros
+// from out-of-range offsets: the count in flight stays fixed, so waits count.
+//
+// The weights are the MFMA's first operand and the tokens the second, so a lane
+// holds four consecutive columns of one token: pairs (gate, up) and (d, d + 32)
+// meet in a lane, and rows leave through the wave's LDS as 16-byte pieces. The
+// 2-byte stores of the transposed form took 14 us per round of 256x256 tiles.
+template <int EPI, int MI, int NI, int WM, int WN, int NS>
+__global__ void __launch_bounds__(64 * WM * WN, 2) pf_gemm(GemmArgs g) {
+  constexpr int NW = WM * WN, AB = MI * WM, BB = NI * WN, NB = AB + BB;   // waves; A, B and all blocks of a k-step
+  constexpr int CPW = (NB + NW - 1) / NW;                                // copies per wave and k-step
+  constexpr bool SPARE = NB % NW != 0;                                   // the last wave's surplus copies
+  constexpr int EROW = 16 * NI * 2 + 16;                                 // bytes of a staged output row (padded)
+  static_assert(NS >= 3 && 16 * EROW * NW <= NS * NB * 1024, "operand ring; staged outputs fit in it");
+  __shared__ u32x4 L[(NS * NB + (SPARE ? 1 : 0)) * 64];
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;   // (uniform: LDS copy bases)
+  // Workgroup w runs on XCD w % 8: each XCD gets a contiguous range of tiles,
+  // rows first, so the workgroups that share weight columns share its L2.
+  const int nt = g.N / (16 * BB), total = g.mt * nt;
+  const int xcd = blockIdx.x & 7, q8 = total >> 3, r8 = total & 7;
+  const int tile = xcd * q8 + min(xcd, r8) + ((int)blockIdx.x >> 3);
+  const int tm = tile % g.mt, tn = tile / g.mt;
+  const int m16 = (g.M + 15) / 16, kb = g.K / 32;
   const rsrc_t ra = make_rsrc(g.a, (size_t)m16 * 16 * g.K * 2);
   const rsrc_t rb = make_rsrc(g.b, (size_t)g.N * g.K * 2);
-  // the k-steps of this workgroup: all of K, or part blockIdx.y of `splits`
-  const int kb = g.K / 32, kn = EPI == EPI_PART ? kb / g.splits : kb;
-  const int k0 = EPI == EPI_PART ? (int)blockIdx.y * kn : 0, ke = k0 + kn;   // kn: a multiple of GEMM_NS
-  // Staging: wave w copies A blocks 2w, 2w+1 and B blocks 2w, 2w+1 of each
-  // k-step from memory straight into LDS (one 1 KiB copy each); k-steps
-  // >= ke copy zeros from out-of-range offsets (no memory read).
-  const int ab0 = tm * 8 + 2 * wave, bb0 = tn * 8 + 2 * wave;
-  auto issue = [&](int ks, int stg) {
-    const bool kin = ks < ke;
+  // the k-steps of this workgroup: all of K, or part blockIdx.y of `splits` (an even number)
+  const int kn = EPI == EPI_PART ? kb / g.splits : kb;
+  const int k0 = EPI == EPI_PART ? (int)blockIdx.y * kn : 0, ke = k0 + kn;
+  // this wave's blocks of a k-step: wave * CPW + u of the A blocks, then the B blocks
+  const uint32_t bstep = g.tiled ? 1024u : 64u;
+  const uint32_t arow = (uint32_t)(lane * 16);
+  const uint32_t brow = g.tiled ? arow : (uint32_t)((lane & 15) * g.K * 2 + (lane >> 4) * 16);
+  uint32_t off[CPW];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const uint32_t ao = kin ? (uint32_t)(((size_t)(ab0 + u) * kb + ks) * 1024 + lane * 16) : OOB;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)&L.st[stg].a[2 * wave + u][0], 16, ao, 0, 0, 0);
-      uint32_t bo = OOB;
-      if (kin)
-        bo = g.tiled ? (uint32_t)(((size_t)(bb0 + u) * kb + ks) * 1024 + lane * 16)
-                     : (uint32_t)((((size_t)(bb0 + u) * 16 + (lane & 15)) * g.K + ks * 32 + (lane >> 4) * 8) * 2);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)&L.st[stg].b[2 * wave + u][0], 16, bo, 0, 0, 0);
+  for (int u = 0; u < CPW; ++u) {
+    const int c = wave * CPW + u;
+    off[u] = c < AB ? arow + (uint32_t)(tm * AB + c) * (uint32_t)kb * 1024u
+                    : brow + (uint32_t)(tn * BB + c - AB) * (uint32_t)kb * 1024u;
+    if (SPARE && c >= NB) off[u] = OOB;
+  }
+  auto issue = [&](int ks, int stg) {
+    const bool in = ks < ke;
+    const uint32_t sa = in ? (uint32_t)ks * 1024u : 0u, sb = in ? (uint32_t)ks * bstep : 0u;
+#pragma unroll
+    for (int u = 0; u < CPW; ++u) {
+      const int c = wave * CPW + u;
+      const lds_ptr_t dst = (lds_ptr_t)&L[(SPARE && c >= NB ? NS * NB : stg * NB + c) * 64];
+      const uint32_t vo = in ? off[u] : OOB;
+      if (c < AB) __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, dst, 16, vo, sa, 0, 0);
+      else __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, dst, 16, vo, sb, 0, 0);
     }
   };
-  // The epilogue's side input, 128 rows of 256 bytes: the RoPE rows of the
-  // tile's tokens (EPI_QKV) or the residual tile (EPI_RES). Two threads per
-  // row load it with 16-byte loads before the first operand copies (so they
-  // are the oldest loads in flight and land first); it goes to LDS after the
-  // k-loop, so the epilogue reads LDS instead of waiting on a 2-byte global
-  // load per element. Rows past the tokens read zero.
-  constexpr bool SIDE = EPI == EPI_QKV || EPI == EPI_RES;
-  const int srow = threadIdx.x >> 1, shalf = threadIdx.x & 1;
-  u32x4 side[SIDE ? 8 : 1];
-  if constexpr (SIDE) {
-    const int m = tm * PF_TM + srow;
-    rsrc_t rs;
-    uint32_t off = OOB;
-    if constexpr (EPI == EPI_RES) {
-      rs = make_rsrc(g.res, (size_t)g.M * g.N * 2);
-      if (m < g.M) off = (uint32_t)(((size_t)m * g.N + (size_t)tn * PF_TN) * 2) + (uint32_t)shalf * 128u;
-    } else {
-      rs = make_rsrc(g.rope, (size_t)g.s_max * (4 * HD));
-      if (m < g.M) off = (uint32_t)((size_t)(g.p0 + m) * (4 * HD)) + (uint32_t)shalf * 128u;
+  // wave (wm, wn) computes rows 16 MI wm .. and columns 16 NI wn .. of the tile
+  const int wm = wave % WM, wn = wave / WM;
+  f32x4 acc[MI][NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 av[2][MI], bv[2][NI];
+  auto read = [&](int stg, u32x4(&a)[MI], u32x4(&b)[NI]) {
+    const u32x4* S = &L[stg * NB * 64 + lane];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) a[i] = S[(MI * wm + i) * 64];
+#pragma unroll
+    for (int j = 0; j < NI; ++j) b[j] = S[(AB + NI * wn + j) * 64];
+  };
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s) issue(k0 + s, s);
+  int stg = 0, fill = NS - 1;
+  wait_copies<(NS - 2) * CPW, 0>();
+  read(0, av[0], bv[0]);
+  for (int ks = k0; ks < ke; ks += 2) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      // k-step ks + s + 1 is in LDS, and every wave has read the stage refilled
+      // next (k-step ks + s - 1's; the MI + NI reads since are ks + s's)
+      wait_copies<(NS - 3) * CPW, MI + NI>();
+      issue(ks + s + NS - 1, fill);
+      fill = stg;
+      stg = stg + 1 == NS ? 0 : stg + 1;
+      read(stg, av[s ^ 1], bv[s ^ 1]);
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) acc[i][j] = mfma16(bv[s][j], av[s][i], acc[i][j]);
+      // one LDS read, then its share of the MFMAs
+      constexpr int R = MI + NI, MM = MI * NI, Q = MM / R, X = MM % R;
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        if (i < X) __builtin_amdgcn_sched_group_barrier(0x008, Q + 1, 0);
+        else if (Q) __builtin_amdgcn_sched_group_barrier(0x008, Q, 0);
+      }
     }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) side[k] = ld16(rs, off == OOB ? OOB : off + 16u * (uint32_t)k);
-  }
-  // wave (wm, wn) computes rows 64*wm .. +63 and columns 64*wn .. +63 of the tile
-  const int wm = wave & 1, wn = wave >> 1;
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int s = 0; s < GEMM_NS - 1; ++s) issue(k0 + s, s);
-  for (int ks = k0; ks < ke; ks += GEMM_NS) {
-#pragma unroll
-    for (int s = 0; s < GEMM_NS; ++s) {
-      // this wave's copies of stage s have landed (the GEMM_NS - 2 later
-      // stages' 4 copies each may be in flight; the side loads, issued
-      // first, have landed too), and, after the barrier, every wave's; every
-      // wave has also finished reading the stage refilled next
-      static_assert(GEMM_NS == 4, "the wait below counts 2 later stages of 4 copies");
-      asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
-      issue(ks + s + GEMM_NS - 1, (s + GEMM_NS - 1) % GEMM_NS);
-      const GemmStage& S = L.st[s];
-      u32x4 av[4], bv[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = S.a[4 * wm + i][lane];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bv[j] = S.b[4 * wn + j][lane];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = mfma16(av[i], bv[j], acc[i][j]);
-    }
-  }
-  const int am = tm * 8 + 4 * wm, bn = tn * 8 + 4 * wn;   // the wave's first A / B tile
-  // the side input into LDS, over the operand stages: every wave's operand
-  // reads and copies (the trailing ones write zeros into the stages) are done
-  const uint16_t* side_lds = reinterpret_cast<const uint16_t*>(&L);   // [PF_TM][SIDE_LD]
-  if constexpr (SIDE) {
-    __syncthreads();
-    u32x4* dst = reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(&L) + srow * SIDE_LD + shalf * 64);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) dst[k] = side[k];
-    __syncthreads();
   }
 
-  // epilogue: acc[i][j][r] is (row 16*(am+i) + 4*(lane/16) + r, column 16*(bn+j) + lane%16)
+  // the ring is free once every wave has read its last operands and its trailing
+  // copies have landed; each wave then stages its rows in a part of its own
+  wait_copies<0, 0>();
+
+  // epilogue: acc[i][j][r] is (row m0(i) + lane%16, column n0 + 16j + 4*(lane/16) + r)
+  const int n0 = 16 * (tn * BB + NI * wn), mw = 16 * (tm * AB + MI * wm);
+  const int lm = lane & 15, lq = lane >> 4;
+  if constexpr (EPI == EPI_PART) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < MI; ++i) {
+      const int m = mw + 16 * i + lm;
+      if (m < g.M)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = 16 * (bn + j) + (lane & 15);
+        for (int j = 0; j < NI; ++j)
+          *reinterpret_cast<f32x4*>(g.part + ((size_t)blockIdx.y * g.M + m) * g.N + n0 + 16 * j + 4 * lq) = acc[i][j];
+    }
+    return;
+  }
+  // (a wave's LDS accesses complete in order; lds_order keeps the compiler's order)
+  auto lds_order = [] { asm volatile("" ::: "memory"); };
+  char* my = reinterpret_cast<char*>(L) + wave * 16 * EROW;
+  if constexpr (EPI == EPI_SWIGLU) {
+    // columns (gate_i, up_i) interleaved: 8 outputs of a token per 16 columns, a
+    // 16-byte slot of the A-tile block (16 tokens x 32 outputs) that 64 columns fill
+    const int kbo = g.N / 64;   // blocks per row of tiles of the output
+    char* out = reinterpret_cast<char*>(g.out) + (size_t)(n0 / 64) * 1024 + (size_t)(n0 % 64) * 16;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = 16 * (am + i) + 4 * (lane >> 4) + r;
-        const float v = acc[i][j][r];
-        if constexpr (EPI == EPI_PART) {
-          if (m < g.M) g.part[((size_t)blockIdx.y * g.M + m) * g.N + n] = v;
-        } else if constexpr (EPI == EPI_RES) {
-          if (m < g.M) {
-            const uint16_t r0 = side_lds[(m - tm * PF_TM) * SIDE_LD + (n - tn * PF_TN)];
-            g.out[(size_t)m * g.N + n] = (uint16_t)f2bf(bf2f(r0) + rbf(v));
-          }
-        } else if constexpr (EPI == EPI_SWIGLU) {
-          // rows (gate_i, up_i) interleaved: lanes 2k (gate) and 2k+1 (up)
-          const float u = dpp<DPP_XOR1>(v);
-          if (m < g.M && (lane & 1) == 0)
-            g.out[a_tile_off(m, n >> 1, g.N / 64)] = (uint16_t)f2bf(v / (1.0f + __expf(-v)) * u);
-        } else {
-          // q, k, v rows in RoPE pairs (d, d+32): lanes 2k (d) and 2k+1 (d+32)
-          const float x = rbf(v);
-          const float y = dpp<DPP_XOR1>(x);
-          if (m < g.M) {
-            const int pair = n >> 1, e = n & 1, pos = g.p0 + m;
-            const int hp = pair & 31;                      // d = hp + 32e
-            const uint16_t* rrow = side_lds + (m - tm * PF_TM) * SIDE_LD;   // row pos of the RoPE table
-            float o = x;
-            if (pair < Q_PAIRS + K_PAIRS) {
-              const float a = e ? y : x, b = e ? x : y;    // the pair (x[d], x[d+32])
-              const int d = hp + 32 * e;
-              const float c = bf2f(rrow[d]), s = bf2f(rrow[HD + d]);
-              o = e ? rbf(rbf(b * c) + rbf(a * s)) : rbf(rbf(a * c) + rbf(-b * s));
-            }
-            const uint16_t ob = (uint16_t)f2bf(o);
-            const int d = hp + 32 * e;
-            if (pair < Q_PAIRS) {
-              g.out[(size_t)m * H + (pair >> 5) * HD + d] = ob;
-            } else if (pair < Q_PAIRS + K_PAIRS) {
-              g.kc[((size_t)((pair - Q_PAIRS) >> 5) * g.s_max + pos) * HD + d] = ob;
-            } else {
-              g.vc[((size_t)((pair - Q_PAIRS - K_PAIRS) >> 5) * g.s_max + pos) * HD + d] = ob;
-            }
+    for (int i = 0; i < MI; ++i) {
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        const f32x4 v = acc[i][j];
+        *reinterpret_cast<uint32_t*>(my + (j * 16 + lm) * 16 + lq * 4) =
+            pack_bf2(v[0] / (1.0f + __expf(-v[0])) * v[1], v[2] / (1.0f + __expf(-v[2])) * v[3]);
+      }
+      lds_order();
+      const int m0 = mw + 16 * i;
+      if (m0 < g.M && lane < 16 * NI)   // (rows past M of the last block: padding of the buffer)
+        *reinterpret_cast<u32x4*>(out + (size_t)(m0 >> 4) * kbo * 1024 + lane * 16) =
+            *reinterpret_cast<const u32x4*>(my + lane * 16);
+      lds_order();
+    }
+  } else {
+    constexpr int PR = 2 * NI, RP = 64 / PR, NP = 16 / RP;   // 16-byte pieces per row, rows per pass, passes
+    const int pc = lane % PR, pr = lane / PR;
+    // QKV: the wave's columns belong to one head (64 columns, RoPE pairs (d, d + 32))
+    const int head = n0 >> 6, d = (n0 & 63) / 2 + 4 * pc;
+    const bool rot = head < NQ + NKV;
+    // the epilogue's side input of up to CI row blocks in flight at once
+    constexpr int CI = MI < 4 ? MI : 4;
+    u32x4 side[EPI == EPI_RES ? CI * NP : 1];
+    uint2 rp[EPI == EPI_QKV ? CI * NP : 1][4];
+    auto load_side = [&](int i0) {
+#pragma unroll
+      for (int i = i0; i < i0 + CI && i < MI; ++i)
+#pragma unroll
+        for (int k = 0; k < NP; ++k) {
+          const int m = mw + 16 * i + k * RP + pr, at = (i - i0) * NP + k;
+          if constexpr (EPI == EPI_RES) {
+            side[at] = u32x4{0u, 0u, 0u, 0u};
+            if (m < g.M) side[at] = *reinterpret_cast<const u32x4*>(g.res + (size_t)m * g.N + n0 + 8 * pc);
+          } else if (rot && m < g.M) {
+            const uint16_t* rrow = g.rope + (size_t)(g.p0 + m) * (2 * HD) + d;   // cos[d], cos[d+32], sin[d], sin[d+32]
+#pragma unroll
+            for (int e = 0; e < 4; ++e) rp[at][e] = *reinterpret_cast<const uint2*>(rrow + 32 * e);
           }
         }
+    };
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      if (i % CI == 0) load_side(i);
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+        *reinterpret_cast<uint2*>(my + lm * EROW + j * 32 + lq * 8) =
+            uint2{pack_bf2(acc[i][j][0], acc[i][j][1]), pack_bf2(acc[i][j][2], acc[i][j][3])};
+      lds_order();
+#pragma unroll
+      for (int k = 0; k < NP; ++k) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(my + (k * RP + pr) * EROW + pc * 16);
+        const int m = mw + 16 * i + k * RP + pr;
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+        if constexpr (EPI == EPI_RES) {
+          const u32x4 r = side[i % CI * NP + k];
+          const uint32_t rw[4] = {r.x, r.y, r.z, r.w};
+          uint32_t o[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = pack_bf2(bf_lo(rw[e]) + bf_lo(w[e]), bf_hi(rw[e]) + bf_hi(w[e]));
+          if (m < g.M) *reinterpret_cast<u32x4*>(g.out + (size_t)m * g.N + n0 + 8 * pc) = u32x4{o[0], o[1], o[2], o[3]};
+        } else if (m < g.M) {
+          float lo[4], hi[4];   // dims d .. d + 3 and d + 32 .. d + 35
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            lo[e] = bf_lo(w[e]);
+            hi[e] = bf_hi(w[e]);
+          }
+          if (rot) {
+            const uint2* R = rp[i % CI * NP + k];
+            const uint32_t c0[2] = {R[0].x, R[0].y}, c1[2] = {R[1].x, R[1].y};
+            const uint32_t s0[2] = {R[2].x, R[2].y}, s1[2] = {R[3].x, R[3].y};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float a = lo[e], b = hi[e];
+              const float ca = e & 1 ? bf_hi(c0[e >> 1]) : bf_lo(c0[e >> 1]), sa = e & 1 ? bf_hi(s0[e >> 1]) : bf_lo(s0[e >> 1]);
+              const float cb = e & 1 ? bf_hi(c1[e >> 1]) : bf_lo(c1[e >> 1]), sb = e & 1 ? bf_hi(s1[e >> 1]) : bf_lo(s1[e >> 1]);
+              lo[e] = rbf(rbf(a * ca) + rbf(-b * sa));
+              hi[e] = rbf(rbf(b * cb) + rbf(a * sb));
+            }
+          }
+          uint16_t* dst;
+          if (head < NQ) dst = g.out + (size_t)m * H + head * HD;
+          else if (rot) dst = g.kc + ((size_t)(head - NQ) * g.s_max + g.p0 + m) * HD;
+          else dst = g.vc + ((size_t)(head - NQ - NKV) * g.s_max + g.p0 + m) * HD;
+          *reinterpret_cast<uint2*>(dst + d) = uint2{pack_bf2(lo[0], lo[1]), pack_bf2(lo[2], lo[3])};
+          *reinterpret_cast<uint2*>(dst + d + 32) = uint2{pack_bf2(hi[0], hi[1]), pack_bf2(hi[2], hi[3])};
+        }
       }
+      lds_order();
     }
   }
 }
 
-// The split-K tail of the O and down projections (N = 2048), one 64-thread
-// workgroup per token row t (the rows spread over every CU): v = the sum of
-// the SPLITS fp32 partials in split order, out = bf16(res + bf16(v))
-// (row-major), and, if xn is given, the next RMSNorm of out into xn (A-tile
-// order), as pf_norm computes it. Every partial of a group of chunks is
-// loaded before the first sum, so the loads overlap instead of waiting one
-// split at a time.
+// The split-K tail of the O and down projections (N = 2048), one workgroup per
+// token row t, 8 columns per thread: v = the sum of the SPLITS fp32 partials in
+// split order, out = bf16(res + bf16(v)) (row-major), and, if xn is given, the
+// next RMSNorm of out into xn (A-tile order), as pf_norm computes it. Latency
+// bounds it: every load of the row is in flight at once (33 tokens of 16 splits
+// on one wave per row, four rounds of loads: 9.4 us).
 template <int SPLITS>
-__global__ void __launch_bounds__(64) pf_reduce_norm(const float* part, const uint16_t* res, uint16_t* out,
+__global__ void __launch_bounds__(NT) pf_reduce_norm(const float* part, const uint16_t* res, uint16_t* out,
                                                      uint16_t* xn, int T) {
-  const int t = blockIdx.x, lane = lane_id();
-  if (t >= T) return;
-  constexpr int CH = SPLITS <= 4 ? 4 : (SPLITS <= 8 ? 2 : 1);   // 512-column chunks loaded at once
-  u32x4 xs[4];
+  static_assert(H == 8 * NT, "8 columns per thread");
+  __shared__ float sums[NWAVE];
+  const int t = blockIdx.x, c = (int)threadIdx.x * 8;
+  float4 pv[SPLITS][2];
 #pragma unroll
-  for (int i0 = 0; i0 < 4; i0 += CH) {
-    float4 pv[CH][SPLITS][2];
-    u32x4 rv[CH];
-#pragma unroll
-    for (int ci = 0; ci < CH; ++ci) {
-      const int c = (i0 + ci) * 512 + lane * 8;
-#pragma unroll
-      for (int sp = 0; sp < SPLITS; ++sp) {
-        const float4* pp = reinterpret_cast<const float4*>(part + ((size_t)sp * T + t) * H + c);
-        pv[ci][sp][0] = pp[0];
-        pv[ci][sp][1] = pp[1];
-      }
-      rv[ci] = *reinterpret_cast<const u32x4*>(res + (size_t)t * H + c);
-    }
-#pragma unroll
-    for (int ci = 0; ci < CH; ++ci) {
-      float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int sp = 0; sp < SPLITS; ++sp) {
-        const float4 p0 = pv[ci][sp][0], p1 = pv[ci][sp][1];
-        v[0] += p0.x; v[1] += p0.y; v[2] += p0.z; v[3] += p0.w;
-        v[4] += p1.x; v[5] += p1.y; v[6] += p1.z; v[7] += p1.w;
-      }
-      const uint32_t rw[4] = {rv[ci].x, rv[ci].y, rv[ci].z, rv[ci].w};
-      uint32_t o[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        o[e] = f2bf(bf_lo(rw[e]) + rbf(v[2 * e])) | (f2bf(bf_hi(rw[e]) + rbf(v[2 * e + 1])) << 16);
-      const int i = i0 + ci;
-      xs[i] = u32x4{o[0], o[1], o[2], o[3]};
-      *reinterpret_cast<u32x4*>(out + (size_t)t * H + i * 512 + lane * 8) = xs[i];
-    }
+  for (int sp = 0; sp < SPLITS; ++sp) {
+    const float4* pp = reinterpret_cast<const float4*>(part + ((size_t)sp * T + t) * H + c);
+    pv[sp][0] = pp[0];
+    pv[sp][1] = pp[1];
   }
-  if (!xn) return;
-  rmsnorm2048(xs, nullptr);
+  const u32x4 rv = *reinterpret_cast<const u32x4*>(res + (size_t)t * H + c);
+  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(xn + a_tile_off(t, i * 512 + lane * 8, H / 32)) = xs[i];
+  for (int sp = 0; sp < SPLITS; ++sp) {
+    const float4 p0 = pv[sp][0], p1 = pv[sp][1];
+    v[0] += p0.x; v[1] += p0.y; v[2] += p0.z; v[3] += p0.w;
+    v[4] += p1.x; v[5] += p1.y; v[6] += p1.z; v[7] += p1.w;
+  }
+  const uint32_t rw[4] = {rv.x, rv.y, rv.z, rv.w};
+  uint32_t o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = pack_bf2(bf_lo(rw[e]) + rbf(v[2 * e]), bf_hi(rw[e]) + rbf(v[2 * e + 1]));
+  *reinterpret_cast<u32x4*>(out + (size_t)t * H + c) = u32x4{o[0], o[1], o[2], o[3]};
+  if (!xn) return;
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) ss = fmaf(bf_hi(o[e]), bf_hi(o[e]), fmaf(bf_lo(o[e]), bf_lo(o[e]), ss));
+  ss = wave_sum(ss);
+  if (lane_id() == 0) sums[wave_id()] = ss;
+  __syncthreads();
+  const float inv = rsqrtf(((sums[0] + sums[1]) + (sums[2] + sums[3])) * (1.0f / H) + EPS);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = cvt_bf2(bf_lo(o[e]) * inv, bf_hi(o[e]) * inv);
+  *reinterpret_cast<u32x4*>(xn + a_tile_off(t, c, H / 32)) = u32x4{o[0], o[1], o[2], o[3]};
 }
 
 // The split-K tail of the QKV projection of short prompts (N = 3072): thread
@@ -498,26 +566,83 @@ __global__ void __launch_bounds__(NT) pf_attn(AttnArgs a) {
 }
 
 size_t ws_per_token() { return (size_t)H * 2 * 5 + (size_t)INTER * 2; }
-// fp32 partials of a split-K projection with N = 2048: splits * M <= 16 * PF_TM rows
-constexpr int PART_ROWS = 16 * PF_TM;
-constexpr size_t PART_BYTES = (size_t)PART_ROWS * H * 4;
+// fp32 partials of a split-K projection: splits * M * N floats in all
+constexpr size_t PART_BYTES = (size_t)2048 * H * 4;
 
-// K splits of an N = 2048 projection over mt row tiles: enough workgroups
-// (16 column tiles each) to occupy the device, 1 when mt alone does it.
-int res_splits(int mt, int kb) {
-  int s = 1;
-  while (mt * s * 2 <= 16 && (kb / (s * 2)) % GEMM_NS == 0) s *= 2;
-  return s;
+// The output tiles pf_gemm is built for: rows, columns, and the time of a
+// launch, fixed + rounds * (round + kstep * k-steps) in us, with one round per
+// 256 workgroups (in fractions above one for the 64x64 tile, three of which
+// share a CU): fitted to launches with weights not in cache over 26 row counts
+// from 16 to 4096 by the four projections' shapes by 1-16 splits (rms error
+// 5-13%). Choosing by it gives up 2% on average against the fastest of nine
+// tiles. (The fixed and round parts are fits, not durations.)
+struct GemmTile {
+  int tm, tn;
+  float fixed, round, kstep;
+};
+constexpr GemmTile TILES[] = {{64, 64, 2.73f, 0.50f, 0.13f},    {128, 128, 0.34f, 5.07f, 0.24f},
+                              {192, 128, -1.88f, 8.42f, 0.32f}, {256, 128, -0.94f, 10.66f, 0.37f},
+                              {192, 128, 8.99f, -0.77f, 0.33f}, {160, 256, 0.30f, 10.96f, 0.45f},
+                              {256, 256, -2.26f, 19.51f, 0.54f}};
+// (built with every epilogue up to here: the others hardly ever win for N = 2048, or with K split)
+constexpr int TILES_RES = 4, TILES_PART = 3, TILES_ALL = sizeof(TILES) / sizeof(TILES[0]);
+
+template <int EPI, int MI, int NI, int WM, int WN, int NS>
+void gemm_launch(const GemmArgs& g, const GemmTile& t, hipStream_t st) {
+  hipLaunchKernelGGL((pf_gemm<EPI, MI, NI, WM, WN, NS>), dim3(g.mt * (g.N / t.tn), g.splits), dim3(64 * WM * WN), 0, st,
+                     g);
+}
+template <int EPI>
+void gemm_run(GemmArgs g, int tile, hipStream_t st) {
+  const GemmTile& t = TILES[tile];
+  g.mt = (g.M + t.tm - 1) / t.tm;
+  switch (tile) {
+    case 0: return gemm_launch<EPI, 2, 2, 2, 2, 6>(g, t, st);
+    case 1: return gemm_launch<EPI, 2, 4, 4, 2, 6>(g, t, st);
+    case 2: return gemm_launch<EPI, 3, 4, 4, 2, 5>(g, t, st);
+  }
+  if constexpr (EPI != EPI_PART) {
+    if (tile == 3) return gemm_launch<EPI, 4, 4, 4, 2, 4>(g, t, st);
+    if constexpr (EPI != EPI_RES) {
+      if (tile == 4) return gemm_launch<EPI, 6, 4, 2, 2, 4>(g, t, st);
+      if (tile == 5) return gemm_launch<EPI, 5, 4, 2, 4, 4>(g, t, st);
+      if (tile == 6) return gemm_launch<EPI, 8, 4, 2, 4, 4>(g, t, st);
+    }
+  }
 }
 
-// K splits of the QKV projection (N = 3072, 24 column tiles) over mt row
-// tiles: up to one round of the 256-CU grid, the partials within PART_BYTES.
-int qkv_splits(int mt) {
-  int s = 1;
-  while (mt * (QKV_ROWS / PF_TN) * s * 2 <= 256 && ((H / 32) / (s * 2)) % GEMM_NS == 0 &&
-         (size_t)s * 2 * mt * PF_TM * QKV_ROWS * 4 <= PART_BYTES)
-    s *= 2;
-  return s;
+// Tile and K splits of a projection of M tokens: the least estimated time, a
+// split's partials and tail included (tail: us of a tail kernel that only a
+// split needs; the partials are written and read once at 3-4 TB/s). An output
+// is the same whatever the tile (its k-steps are summed in order) but not
+// whatever the split, so the splits are those of M rounded up to 128 tokens
+// (of 64 for the first 128, where short turns lie): a prompt of up to 128
+// tokens gives the same bits in any chunks.
+struct GemmPlan {
+  int tile, splits;
+};
+float gemm_us(const GemmTile& t, int M, int N, int K, int splits, float tail) {
+  const int wg = (M + t.tm - 1) / t.tm * (N / t.tn) * splits;
+  const float rounds = t.tm == 64 ? fmaxf(1.f, (float)wg / 256.f) : (float)((wg + 255) / 256);
+  const float us = t.fixed + rounds * (t.round + t.kstep * (float)(K / 32 / splits));
+  return splits == 1 ? us : us + tail + (float)splits * (float)M * (float)N * 4.f / 7e6f;
+}
+GemmPlan gemm_plan(int M, int N, int K, int tiles, bool split, float tail) {
+  GemmPlan best = {0, 1};
+  const int most = (M + 127) / 128 * 128, Ms = most <= 128 ? 64 : most;
+  for (int sp = 2; split && sp <= 16 && (size_t)sp * most * N * 4 <= PART_BYTES; sp *= 2) {
+    auto least = [&](int s) {
+      const int n = s > 1 ? TILES_PART : tiles;
+      float us = gemm_us(TILES[0], Ms, N, K, s, tail);
+      for (int i = 1; i < n; ++i) us = fminf(us, gemm_us(TILES[i], Ms, N, K, s, tail));
+      return us;
+    };
+    if (least(sp) < least(best.splits)) best.splits = sp;
+  }
+  const int n = best.splits > 1 ? TILES_PART : tiles;
+  for (int i = 1; i < n; ++i)
+    if (gemm_us(TILES[i], M, N, K, best.splits, tail) < gemm_us(TILES[best.tile], M, N, K, best.splits, tail)) best.tile = i;
+  return best;
 }
 
 }  // namespace
@@ -554,29 +679,28 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
   const int L = a->n_layers, l0 = a->first_layer;
   // An N = 2048 projection (O: K = 2048, down: K = 8192) of T tokens with the
   // residual add, followed by the RMSNorm of its output into xn if `norm`:
-  // as one GEMM with the add in its epilogue plus pf_norm when its 16 x mt
-  // workgroups occupy the device, else split over K into fp32 partials that
+  // as one GEMM with the add in its epilogue plus pf_norm, or, where few tiles
+  // would leave the device idle, split over K into fp32 partials that
   // pf_reduce_norm sums (in split order), adds and normalises.
-  auto res_gemm = [&](GemmArgs g, const uint16_t* res, uint16_t* out, bool norm, int T, int mt) {
-    const int sp = res_splits(mt, g.K / 32);
-    const dim3 tg((unsigned)((T + NWAVE - 1) / NWAVE));
-    if (sp == 1) {
+  auto res_gemm = [&](GemmArgs g, const uint16_t* res, uint16_t* out, bool norm, int T) {
+    const GemmPlan pl = gemm_plan(T, g.N, g.K, TILES_RES, true, -0.5f);
+    g.splits = pl.splits;
+    if (pl.splits == 1) {
       g.res = res;
       g.out = out;
-      hipLaunchKernelGGL(pf_gemm<EPI_RES>, dim3(mt * (H / PF_TN)), dim3(NT), 0, st, g);
+      gemm_run<EPI_RES>(g, pl.tile, st);
       if (norm)
-        hipLaunchKernelGGL(pf_norm, tg, dim3(NT), 0, st, (const uint16_t*)out, (const int32_t*)nullptr,
-                           (const uint16_t*)nullptr, (uint16_t*)nullptr, xn, T);
+        hipLaunchKernelGGL(pf_norm, dim3((unsigned)((T + NWAVE - 1) / NWAVE)), dim3(NT), 0, st, (const uint16_t*)out,
+                           (const int32_t*)nullptr, (const uint16_t*)nullptr, (uint16_t*)nullptr, xn, T);
     } else {
-      g.splits = sp;
       g.part = part;
-      hipLaunchKernelGGL(pf_gemm<EPI_PART>, dim3(mt * (H / PF_TN), sp), dim3(NT), 0, st, g);
+      gemm_run<EPI_PART>(g, pl.tile, st);
       uint16_t* xn_out = norm ? xn : nullptr;
-      switch (sp) {   // res_splits gives 2, 4, 8 or 16
-        case 2: hipLaunchKernelGGL(pf_reduce_norm<2>, dim3(T), dim3(64), 0, st, (const float*)part, res, out, xn_out, T); break;
-        case 4: hipLaunchKernelGGL(pf_reduce_norm<4>, dim3(T), dim3(64), 0, st, (const float*)part, res, out, xn_out, T); break;
-        case 8: hipLaunchKernelGGL(pf_reduce_norm<8>, dim3(T), dim3(64), 0, st, (const float*)part, res, out, xn_out, T); break;
-        default: hipLaunchKernelGGL(pf_reduce_norm<16>, dim3(T), dim3(64), 0, st, (const float*)part, res, out, xn_out, T); break;
+      switch (pl.splits) {   // gemm_plan gives 2, 4, 8 or 16
+        case 2: hipLaunchKernelGGL(pf_reduce_norm<2>, dim3(T), dim3(NT), 0, st, (const float*)part, res, out, xn_out, T); break;
+        case 4: hipLaunchKernelGGL(pf_reduce_norm<4>, dim3(T), dim3(NT), 0, st, (const float*)part, res, out, xn_out, T); break;
+        case 8: hipLaunchKernelGGL(pf_reduce_norm<8>, dim3(T), dim3(NT), 0, st, (const float*)part, res, out, xn_out, T); break;
+        default: hipLaunchKernelGGL(pf_reduce_norm<16>, dim3(T), dim3(NT), 0, st, (const float*)part, res, out, xn_out, T); break;
       }
     }
   };
@@ -585,7 +709,6 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
   // only its QKV GEMM unless the hidden state is asked for.
   for (int c0 = 0; c0 < a->n_tokens; c0 += cap) {
     const int T = min(cap, a->n_tokens - c0), p0 = a->start_pos + c0;
-    const int mt = (T + PF_TM - 1) / PF_TM;
     hipLaunchKernelGGL(pf_norm, dim3((T + NWAVE - 1) / NWAVE), dim3(NT), 0, st, (const uint16_t*)nullptr,
                        a->tokens + c0, static_cast<const uint16_t*>(w->embed), x, xn, T);
     for (int li = 0; li < L; ++li) {
@@ -609,18 +732,20 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
       g.out = q;
       g.kc = kc;
       g.vc = vc;
-      const int qs = qkv_splits(mt);
-      if (qs == 1) {
-        hipLaunchKernelGGL(pf_gemm<EPI_QKV>, dim3(mt * (QKV_ROWS / PF_TN)), dim3(NT), 0, st, g);
+      const GemmPlan qp = gemm_plan(T, QKV_ROWS, H, TILES_ALL, true, 4.5f);
+      g.splits = qp.splits;
+      if (qp.splits == 1) {
+        gemm_run<EPI_QKV>(g, qp.tile, st);
       } else {   // short prompts: split over K, RoPE and the scatter in the tail
-        g.splits = qs;
         g.part = part;
-        hipLaunchKernelGGL(pf_gemm<EPI_PART>, dim3(mt * (QKV_ROWS / PF_TN), qs), dim3(NT), 0, st, g);
+        gemm_run<EPI_PART>(g, qp.tile, st);
         const uint16_t* rope = static_cast<const uint16_t*>(w->rope);
-        switch (qs) {   // qkv_splits gives 2, 4 or 8
-          case 2: hipLaunchKernelGGL(pf_qkv_finish<2>, dim3(T, QKV_PAIRS / 2 / NT), dim3(NT), 0, st, (const float*)part, rope, q, kc, vc, T, p0, a->s_max); break;
-          case 4: hipLaunchKernelGGL(pf_qkv_finish<4>, dim3(T, QKV_PAIRS / 2 / NT), dim3(NT), 0, st, (const float*)part, rope, q, kc, vc, T, p0, a->s_max); break;
-          default: hipLaunchKernelGGL(pf_qkv_finish<8>, dim3(T, QKV_PAIRS / 2 / NT), dim3(NT), 0, st, (const float*)part, rope, q, kc, vc, T, p0, a->s_max); break;
+        const dim3 fg(T, QKV_PAIRS / 2 / NT);
+        switch (qp.splits) {   // gemm_plan gives 2, 4, 8 or 16
+          case 2: hipLaunchKernelGGL(pf_qkv_finish<2>, fg, dim3(NT), 0, st, (const float*)part, rope, q, kc, vc, T, p0, a->s_max); break;
+          case 4: hipLaunchKernelGGL(pf_qkv_finish<4>, fg, dim3(NT), 0, st, (const float*)part, rope, q, kc, vc, T, p0, a->s_max); break;
+          case 8: hipLaunchKernelGGL(pf_qkv_finish<8>, fg, dim3(NT), 0, st, (const float*)part, rope, q, kc, vc, T, p0, a->s_max); break;
+          default: hipLaunchKernelGGL(pf_qkv_finish<16>, fg, dim3(NT), 0, st, (const float*)part, rope, q, kc, vc, T, p0, a->s_max); break;
         }
         g.splits = 1;
       }
@@ -640,25 +765,23 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
       g.N = H;
       g.K = H;
       g.kc = g.vc = nullptr;
-      res_gemm(g, x, h1, true, T, mt);
+      res_gemm(g, x, h1, true, T);
       // gate/up + SwiGLU -> act
       g.a = xn;
       g.b = Wgu + (size_t)l * 2 * INTER * H;
       g.N = 2 * INTER;
       g.K = H;
       g.out = act;
-      hipLaunchKernelGGL(pf_gemm<EPI_SWIGLU>, dim3(mt * (2 * INTER / PF_TN)), dim3(NT), 0, st, g);
-      // down projection + residual -> x (the next layer's input), its RMSNorm -> xn
+      g.splits = 1;
+      gemm_run<EPI_SWIGLU>(g, gemm_plan(T, g.N, g.K, TILES_ALL, false, 0.f).tile, st);
+      // down projection + residual -> x (the next layer's input) and its RMSNorm -> xn,
+      // or the caller's hidden state after the last layer
       g.a = act;
       g.b = Wd + (size_t)l * H * INTER;
       g.N = H;
       g.K = INTER;
-      res_gemm(g, h1, x, li + 1 < L, T, mt);
-    }
-    if (a->hidden_out) {
-      const hipError_t e = hipMemcpyAsync(static_cast<uint16_t*>(a->hidden_out) + (size_t)c0 * H, x,
-                                          (size_t)T * H * 2, hipMemcpyDeviceToDevice, st);
-      if (e != hipSuccess) return e;
+      if (li + 1 < L) res_gemm(g, h1, x, true, T);
+      else res_gemm(g, h1, static_cast<uint16_t*>(a->hidden_out) + (size_t)c0 * H, false, T);
     }
   }
   return hipGetLastError();
