@@ -47,7 +47,8 @@ namespace {
 
 using namespace mk;
 
-constexpr int PF_TB = 16;                 // tokens per attention workgroup
+// fp32 partials: a projection's (splits * M * N floats) or the attention's key splits
+constexpr size_t PART_BYTES = (size_t)2048 * H * 4;
 
 enum : int { EPI_QKV = 0, EPI_RES = 1, EPI_SWIGLU = 2, EPI_PART = 3 };
 
@@ -433,142 +434,272 @@ struct AttnArgs {
   const uint16_t* kc;    // the layer's caches bf16 [8][s_max][64]
   const uint16_t* vc;
   uint16_t* att;         // A-tile order [T16][2048]
+  float* part;           // key splits: o of (split, token, q head) [64], then (max, sum) of each
   int T, p0, s_max;
+  int split;             // keys per split (a multiple of KB)
+  int nsplit;
 };
 
-constexpr int KS_STRIDE = HD + 8;   // K tile row in LDS (bf16): 144 bytes, rows on distinct banks
-constexpr int VT_STRIDE = 32 + 4;   // transposed V tile row (one dim, 32 keys): 72 bytes
+constexpr int KB = 64;                // keys per step
+constexpr int VT_LD = KB + 8;         // bf16 per row (one dim) of the transposed V tile: 144 bytes
+constexpr int ANS = 3;                // steps of K and V in LDS
+constexpr float QK_LOG2 = SM_SCALE * 1.4426950408889634f;   // scores in units of log2: p = 2^(s - max)
 
-struct AttnLds {
-  uint16_t k[2][32][KS_STRIDE];
-  uint16_t vt[2][HD][VT_STRIDE];
+// K and V of one step in LDS: K as 8 blocks of 1 KiB, (16 keys x 32 dims) in
+// the MFMA's operand order (a_tile_off's), block 2 * (key / 16) + dim / 32; V
+// transposed, the keys of a 32-key half in the order of the MFMA's k-slots (the
+// 8 slots of lane group q4 are keys 4 q4 + i and 16 + 4 q4 + i, as p is held).
+struct AttnTile {
+  u32x4 k[8][64];
+  uint16_t vt[HD][VT_LD];
 };
 
-// Token t of the sequence (position p0 + t) attends to cache rows [0, p0 + t],
-// its own row included (written by the QKV GEMM before this launch).
-__global__ void __launch_bounds__(NT) pf_attn(AttnArgs a) {
-  __shared__ AttnLds L;
-  const int tid = threadIdx.x, wave = wave_id(), lane = lane_id();
-  const int nblk = (a.T + PF_TB - 1) / PF_TB;
-  const int tb = nblk - 1 - (int)blockIdx.x;   // the longest blocks first
-  const int g = blockIdx.y;                    // kv head
-  const int t0 = tb * PF_TB;
-  const int n_keys = a.p0 + min(t0 + PF_TB, a.T);
-  // this lane's column: token t0 + 4*wave + (lane%16)/4, q head 4g + lane%4
-  const int col = lane & 15, q4 = lane >> 4;
-  const int tq = t0 + 4 * wave + (col >> 2);
-  const int hq = GQA * g + (col & 3);
-  const int lim = a.p0 + min(tq, a.T - 1);     // last key of the column (padding tokens: any finite row)
+// Causal attention. Token t of the sequence (position p0 + t) attends to cache
+// rows [0, p0 + t], its own row included (written by the QKV projection before
+// this launch). A workgroup takes 16 NTL tokens of one kv head, wave h the
+// group's q head h, NTL tiles of 16 tokens; SPLIT: one range of keys of them,
+// its unnormalised output to `part` for pf_attn_merge.
+//
+// What bounds it: with many workgroups the exponentials (16 cycles each for a
+// wave) and the operations around them, 28 cycles per 64 scores against 16 of
+// MFMA; so the scale and the maximum go into one fma, masks are applied only on
+// the diagonal, the accumulators are rescaled only when a maximum moved, and a
+// step is 64 keys. With few, memory latency and what one CU can read: K goes
+// from memory straight into LDS two steps ahead, V is loaded two steps ahead and
+// transposed into LDS one step ahead, four keys by four dims at a time (one
+// 8-byte store per dim). Workgroup w runs on XCD w % 8, which is its kv head: a
+// head's K and V are read into one L2. Within a head the longest come first.
+// Measured against 16-token workgroups with 32-key steps, one step ahead, and V
+// transposed by 2-byte stores: 3001 tokens 112 -> 69 us, 1100 tokens 28.8 -> 23.
+// Three and four tiles per wave are slower than two (84 and 94 us at 3001).
+template <int NTL, bool SPLIT>
+__global__ void __launch_bounds__(NT, NTL > 2 ? 2 : 3) pf_attn(AttnArgs a) {
+  __shared__ AttnTile L[ANS];
+  const int h = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), tid_ = threadIdx.x, lane = tid_ & 63;
+  const int nblk = (a.T + 16 * NTL - 1) / (16 * NTL);
+  const int g = blockIdx.x & 7;                // kv head
+  static_assert(NKV == 8, "a kv head per XCD");
+  const int tb = nblk - 1 - ((int)blockIdx.x >> 3) % nblk, sp = ((int)blockIdx.x >> 3) / nblk;
+  const int t0 = tb * 16 * NTL;
+  const int k_end = a.p0 + min(t0 + 16 * NTL, a.T);
+  const int key0 = SPLIT ? sp * a.split : 0, n_keys = SPLIT ? min(k_end, key0 + a.split) : k_end;
+  if (SPLIT && key0 >= k_end) return;          // (the merge knows)
+  const int col = lane & 15, q4 = lane >> 4, hq = GQA * g + h;
   const rsrc_t rq = make_rsrc(a.q, (size_t)a.T * H * 2);
-  u32x4 qv[2];
+  u32x4 qv[NTL][2];   // this lane's token: t0 + 16 j + col
 #pragma unroll
-  for (int s = 0; s < 2; ++s)
-    qv[s] = ld16(rq, tq < a.T ? (uint32_t)(((size_t)tq * H + hq * HD + 32 * s + q4 * 8) * 2) : OOB);
+  for (int j = 0; j < NTL; ++j)
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int tq = t0 + 16 * j + col;
+      qv[j][s] = ld16(rq, tq < a.T ? (uint32_t)(((size_t)tq * H + hq * HD + 32 * s + q4 * 8) * 2) : OOB);
+    }
   const rsrc_t rk = make_rsrc(a.kc + (size_t)g * a.s_max * HD, (size_t)a.s_max * HD * 2);
   const rsrc_t rv = make_rsrc(a.vc + (size_t)g * a.s_max * HD, (size_t)a.s_max * HD * 2);
-  // staging of a 32-key block: thread t loads key row t/8, dims (t%8)*8 .. +7 of K and of V
-  const int sr = tid >> 3, sc = tid & 7;
-  auto load_blk = [&](int kb, u32x4& kk, u32x4& vv) {
-    const int key = kb * 32 + sr;
-    const uint32_t off = key < n_keys ? (uint32_t)((key * HD + sc * 8) * 2) : OOB;
-    kk = ld16(rk, off);
-    vv = ld16(rv, off);
+  // Staging: wave h copies K blocks 2h and 2h + 1 (keys 16 h + lane%16); thread
+  // t loads V rows 4 (t/16) .. + 3, dims 4 (t%16) .. + 3. Keys past the range
+  // read zero (no memory access), so the number in flight is fixed.
+  const int vk = (tid_ >> 4) * 4, vd = (tid_ & 15) * 4;
+  auto stage_k = [&](int k0, AttnTile& t) {
+    const int key = k0 + 16 * h + col;
+    const uint32_t off = key < n_keys ? (uint32_t)((key * HD + q4 * 8) * 2) : OOB;
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_ptr_t)&t.k[2 * h + s][0], 16, off + 64u * s, 0, 0, 0);
   };
-  auto store_blk = [&](int buf, const u32x4& kk, const u32x4& vv) {
-    *reinterpret_cast<u32x4*>(&L.k[buf][sr][sc * 8]) = kk;
-    const uint32_t w[4] = {vv.x, vv.y, vv.z, vv.w};
+  auto load_v = [&](int k0, uint2 (&v)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int key = k0 + vk + i;
+      const auto w = __builtin_amdgcn_raw_buffer_load_b64(rv, key < n_keys ? (int)((key * HD + vd) * 2) : (int)OOB, 0, 0);
+      v[i] = uint2{(uint32_t)w[0], (uint32_t)w[1]};
+    }
+  };
+  auto store_v = [&](const uint2 (&v)[4], AttnTile& t) {
+    // keys vk .. + 3 of dim vd + e, at the k-slots of keys vk % 32 .. + 3
+    const int slot = (vk & 32) + ((vk & 15) >> 2) * 8 + ((vk >> 4) & 1) * 4;
+    const uint32_t lo[4] = {v[0].x, v[1].x, v[2].x, v[3].x}, hi[4] = {v[0].y, v[1].y, v[2].y, v[3].y};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      L.vt[buf][sc * 8 + 2 * e][sr] = (uint16_t)(w[e] & 0xffffu);
-      L.vt[buf][sc * 8 + 2 * e + 1][sr] = (uint16_t)(w[e] >> 16);
+      const uint32_t* w = e < 2 ? lo : hi;
+      const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;   // the upper or the lower halves of two words
+      *reinterpret_cast<uint2*>(&t.vt[vd + e][slot]) =
+          uint2{__builtin_amdgcn_perm(w[1], w[0], sel), __builtin_amdgcn_perm(w[3], w[2], sel)};
     }
   };
-  const int nb = (n_keys + 31) / 32;
-  {
-    u32x4 kk, vv;
-    load_blk(0, kk, vv);
-    store_blk(0, kk, vv);
+  f32x4 acc[NTL][4];
+  float m_run[NTL], l_run[NTL];
+#pragma unroll
+  for (int j = 0; j < NTL; ++j) {
+    m_run[j] = -INFINITY;
+    l_run[j] = 0.f;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) acc[j][d] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  __syncthreads();
-  f32x4 acc[4];
+  auto compute = [&](int k0, const AttnTile& cur) {
+    // S^T: keys 16 kt + 4 q4 + i of the step, this lane's token of each tile
+    f32x4 s[NTL][4];
 #pragma unroll
-  for (int d = 0; d < 4; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
-  for (int kb = 0; kb < nb; ++kb) {
-    const int buf = kb & 1;
-    u32x4 kk, vv;
-    const bool more = kb + 1 < nb;
-    if (more) load_blk(kb + 1, kk, vv);
-    // S^T: keys 16*ks + 4*q4 + i of the block, this lane's column
-    float sc4[2][4];
-    float mb = -INFINITY;
+    for (int kt = 0; kt < 4; ++kt) {
+      const u32x4 ka = cur.k[2 * kt][lane], kb = cur.k[2 * kt + 1][lane];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < NTL; ++j)
+        s[j][kt] = mfma16(kb, qv[j][1], mfma16(ka, qv[j][0], f32x4{0.f, 0.f, 0.f, 0.f}));
+    }
+    u32x4 pb[NTL][2];
 #pragma unroll
-      for (int sd = 0; sd < 2; ++sd) {
-        const u32x4 ko = *reinterpret_cast<const u32x4*>(&L.k[buf][16 * ks + col][32 * sd + q4 * 8]);
-        s = mfma16(ko, qv[sd], s);
+    for (int j = 0; j < NTL; ++j) {
+      if (k0 + KB - 1 > a.p0 + t0 + 16 * j) {   // keys past some token of the tile
+        const int lim = a.p0 + min(t0 + 16 * j + col, a.T - 1);   // (padding tokens: any finite row)
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (k0 + 16 * kt + 4 * q4 + i > lim) s[j][kt][i] = -INFINITY;
       }
+      float mb = fmaxf(fmaxf(s[j][0][0], s[j][0][1]), fmaxf(s[j][0][2], s[j][0][3]));
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int key = kb * 32 + 16 * ks + 4 * q4 + i;
-        const float v = key <= lim ? s[i] * SM_SCALE : -INFINITY;
-        sc4[ks][i] = v;
-        mb = fmaxf(mb, v);
+      for (int kt = 1; kt < 4; ++kt)
+        mb = fmaxf(mb, fmaxf(fmaxf(s[j][kt][0], s[j][kt][1]), fmaxf(s[j][kt][2], s[j][kt][3])));
+      mb = max_xor32(max_xor16(mb)) * QK_LOG2;   // the token's maximum over the step
+      const float m_new = fmaxf(m_run[j], mb);
+      const float m_use = SPLIT && m_new == -INFINITY ? 0.f : m_new;   // (a split's keys may all be masked)
+      if (__any(m_new != m_run[j])) {
+        const float alpha = __builtin_amdgcn_exp2f(m_run[j] - m_use);
+        l_run[j] *= alpha;
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[j][d][i] *= alpha;
+        m_run[j] = m_new;
+      }
+      float p[4][4];
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[kt][i] = __builtin_amdgcn_exp2f(fmaf(s[j][kt][i], QK_LOG2, -m_use));
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) l_run[j] += (p[kt][0] + p[kt][1]) + (p[kt][2] + p[kt][3]);
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+        pb[j][hf] = u32x4{cvt_bf2(p[2 * hf][0], p[2 * hf][1]), cvt_bf2(p[2 * hf][2], p[2 * hf][3]),
+                          cvt_bf2(p[2 * hf + 1][0], p[2 * hf + 1][1]), cvt_bf2(p[2 * hf + 1][2], p[2 * hf + 1][3])};
+    }
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const u32x4 vo = *reinterpret_cast<const u32x4*>(&cur.vt[16 * d + col][32 * hf + 8 * q4]);
+#pragma unroll
+        for (int j = 0; j < NTL; ++j) acc[j][d] = mfma16(vo, pb[j][hf], acc[j][d]);
+      }
+  };
+  // Step i: its K copies and V loads are issued two steps before, V goes to LDS
+  // one step before. Every wait leaves the 6 loads of the latest step in flight.
+  constexpr int FLY = 6;
+  uint2 v[2][4];
+  load_v(key0, v[0]);
+  stage_k(key0, L[0]);
+  load_v(key0 + KB, v[1]);
+  stage_k(key0 + KB, L[1]);
+  store_v(v[0], L[0]);
+  wait_copies<FLY, 0>();
+  const int steps = (n_keys - key0 + KB - 1) / KB;
+  int slot = 0;
+  for (int it = 0; it < steps; it += 2) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (it + u < steps) {
+        const int k0 = key0 + (it + u) * KB, s1 = slot == ANS - 1 ? 0 : slot + 1, s2 = s1 == ANS - 1 ? 0 : s1 + 1;
+        load_v(k0 + 2 * KB, v[u]);
+        stage_k(k0 + 2 * KB, L[s2]);
+        compute(k0, L[slot]);
+        store_v(v[u ^ 1], L[s1]);
+        wait_copies<FLY, 0>();
+        slot = s1;
       }
     }
-    mb = max_xor32(max_xor16(mb));          // the column's maximum over the 32 keys
-    const float m_new = fmaxf(m_run, mb);   // finite: key 0 is in every column's range
-    const float alpha = __expf(m_run - m_new);
-    m_run = m_new;
-    float ps = 0.f;
-    float p[2][4];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        p[ks][i] = __expf(sc4[ks][i] - m_new);
-        ps += p[ks][i];
-      }
-    l_run = l_run * alpha + ps;
-    // P^T as the B operand: k-slots 8*q4 .. +7 of lane (q4, col) are the keys
-    // 4*q4 + i and 16 + 4*q4 + i it holds (the V^T operand uses the same key order)
-    const u32x4 pb = {cvt_bf2(p[0][0], p[0][1]), cvt_bf2(p[0][2], p[0][3]), cvt_bf2(p[1][0], p[1][1]),
-                      cvt_bf2(p[1][2], p[1][3])};
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const uint16_t* vrow = &L.vt[buf][16 * d + col][0];
-      const uint2 lo = *reinterpret_cast<const uint2*>(vrow + 4 * q4);
-      const uint2 hi = *reinterpret_cast<const uint2*>(vrow + 16 + 4 * q4);
-      const u32x4 vo = {lo.x, lo.y, hi.x, hi.y};
-      f32x4 c = acc[d];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) c[i] *= alpha;
-      acc[d] = mfma16(vo, pb, c);
-    }
-    if (more) store_blk(buf ^ 1, kk, vv);
-    __syncthreads();
   }
-  // the column's sum over its four lanes; o = acc / l, dims 16d + 4*q4 + i
-  const float l_tot = add_xor32(add_xor16(l_run));
-  const float inv = 1.0f / l_tot;
-  if (tq < a.T) {
+  // the token's sum over its four lanes; o = acc / l, dims 16 d + 4 q4 + i
 #pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const int dim = 16 * d + 4 * q4;
-      uint2 w;
-      w.x = pack_bf2(acc[d][0] * inv, acc[d][1] * inv);
-      w.y = pack_bf2(acc[d][2] * inv, acc[d][3] * inv);
-      *reinterpret_cast<uint2*>(a.att + a_tile_off(tq, hq * HD + dim, H / 32)) = w;
+  for (int j = 0; j < NTL; ++j) {
+    const int tq = t0 + 16 * j + col;
+    const float l_tot = add_xor32(add_xor16(l_run[j]));
+    if (tq >= a.T) continue;
+    if constexpr (SPLIT) {
+      const size_t at = ((size_t)sp * a.T + tq) * NQ + hq, n = (size_t)a.nsplit * a.T * NQ;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) *reinterpret_cast<f32x4*>(a.part + at * HD + 16 * d + 4 * q4) = acc[j][d];
+      if (q4 == 0) *reinterpret_cast<float2*>(a.part + n * HD + at * 2) = float2{m_run[j], l_tot};
+    } else {
+      const float inv = 1.0f / l_tot;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        uint2 w;
+        w.x = pack_bf2(acc[j][d][0] * inv, acc[j][d][1] * inv);
+        w.y = pack_bf2(acc[j][d][2] * inv, acc[j][d][3] * inv);
+        *reinterpret_cast<uint2*>(a.att + a_tile_off(tq, hq * HD + 16 * d + 4 * q4, H / 32)) = w;
+      }
     }
   }
 }
 
-size_t ws_per_token() { return (size_t)H * 2 * 5 + (size_t)INTER * 2; }
-// fp32 partials of a split-K projection: splits * M * N floats in all
-constexpr size_t PART_BYTES = (size_t)2048 * H * 4;
+// The attention output from the splits' parts: 16 lanes per (token, q head),
+// four dims each; the splits that hold keys of the token's workgroup, in order.
+__global__ void __launch_bounds__(NT) pf_attn_merge(AttnArgs a, int tokens_per_wg) {
+  const int i = (int)blockIdx.x * (NT / 16) + ((int)threadIdx.x >> 4), t = i / NQ, hq = i % NQ;
+  const int d = ((int)threadIdx.x & 15) * 4;
+  if (t >= a.T) return;
+  const int k_end = a.p0 + min((t / tokens_per_wg + 1) * tokens_per_wg, a.T);
+  const int ns = min((k_end + a.split - 1) / a.split, a.nsplit);
+  const float2* ml = reinterpret_cast<const float2*>(a.part + (size_t)a.nsplit * a.T * NQ * HD);
+  float M = -INFINITY;
+  for (int s = 0; s < ns; ++s) M = fmaxf(M, ml[((size_t)s * a.T + t) * NQ + hq].x);
+  float l = 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < ns; ++s) {
+    const size_t at = ((size_t)s * a.T + t) * NQ + hq;
+    const float2 x = ml[at];
+    const float f = __builtin_amdgcn_exp2f(x.x - M);
+    l = fmaf(x.y, f, l);
+    o += *reinterpret_cast<const f32x4*>(a.part + at * HD + d) * f;
+  }
+  const float inv = 1.0f / l;
+  *reinterpret_cast<uint2*>(a.att + a_tile_off(t, hq * HD + d, H / 32)) =
+      uint2{pack_bf2(o[0] * inv, o[1] * inv), pack_bf2(o[2] * inv, o[3] * inv)};
+}
 
+template <int NTL, bool SPLIT>
+void attn_launch(const AttnArgs& a, hipStream_t st) {
+  const int nblk = (a.T + 16 * NTL - 1) / (16 * NTL);
+  hipLaunchKernelGGL((pf_attn<NTL, SPLIT>), dim3(nblk * NKV * (SPLIT ? a.nsplit : 1)), dim3(NT), 0, st, a);
+  if (SPLIT) hipLaunchKernelGGL(pf_attn_merge, dim3((a.T * NQ + NT / 16 - 1) / (NT / 16)), dim3(NT), 0, st, a, 16 * NTL);
+}
+// Tiles of 16 tokens up to 2048 tokens, of 32 above (one 16-token tile per wave
+// against two: 2048 tokens 44 against 47 us, 3001 tokens 92 against 71). Few
+// workgroups over many keys split them, up to 8 ways, as far as the device has
+// room for (three workgroups per CU) and the partials fit: a step of 64 keys
+// takes one workgroup 0.85 us, the parts and the merge 5 us and what they move
+// (33 tokens at 4000 rows: 55 us whole, 17.5 in 8 parts; at 700 rows 13.6 and
+// 11.0). Splits begin at multiples of 64 keys of the cache.
+void attn_run(AttnArgs a, hipStream_t st) {
+  const int n_keys = a.p0 + a.T, wgs = (a.T + 15) / 16 * NKV;
+  const int most = (int)(PART_BYTES / ((size_t)NQ * (HD + 2) * 4)) / a.T;   // splits whose parts fit
+  const int ns = min(min(8, 3 * 256 / wgs), most);
+  if (ns >= 2) {
+    const int split = max(4 * KB, (n_keys + ns * KB - 1) / (ns * KB) * KB);
+    const float saved = (float)(n_keys - split) / KB * 0.85f;
+    if (saved > 5.f + (float)(ns * a.T) * (NQ * (HD + 2) * 4) * 2.f / 4e6f) {
+      a.split = split;
+      a.nsplit = (n_keys + split - 1) / split;
+      return attn_launch<1, true>(a, st);
+    }
+  }
+  if (a.T <= 2048) attn_launch<1, false>(a, st);
+  else attn_launch<2, false>(a, st);
+}
+
+size_t ws_per_token() { return (size_t)H * 2 * 5 + (size_t)INTER * 2; }
 // The output tiles pf_gemm is built for: rows, columns, and the time of a
 // launch, fixed + rounds * (round + kstep * k-steps) in us, with one round per
 // 256 workgroups (in fractions above one for the 64x64 tile, three of which
@@ -755,10 +886,11 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
       aa.kc = kc;
       aa.vc = vc;
       aa.att = att;
+      aa.part = part;
       aa.T = T;
       aa.p0 = p0;
       aa.s_max = a->s_max;
-      hipLaunchKernelGGL(pf_attn, dim3((T + PF_TB - 1) / PF_TB, NKV), dim3(NT), 0, st, aa);
+      attn_run(aa, st);
       // O projection + residual -> h1, its RMSNorm -> xn
       g.a = att;
       g.b = Wo + (size_t)l * H * H;

@@ -1,9 +1,12 @@
 """GPU parity of one prefill layer (``mk_prefill`` with the hidden state out)
-at row counts around the edges of its GEMM tiles and K splits.
+at row counts around the edges of its GEMM tiles and K splits, and behind
+caches long enough for its attention to split the keys.
 
 The projections run on output tiles from 64x64 to 256x256, with K split into
 partials for short prompts, chosen by row count; the counts here lie on both
-sides of the tiles' and the splits' edges and reach every tile. For each:
+sides of the tiles' and the splits' edges and reach every tile. The attention
+takes 16 or 32 tokens per workgroup in steps of 64 keys and, for few tokens
+behind many rows, splits the keys over workgroups. For each count and start:
 
 * the hidden state and the K/V rows against plain torch on the GPU: fp32
   products with bf16 rounding at the kernel's points ("rounded") and float64
@@ -24,7 +27,8 @@ from gpu_common import need_gpu, say
 
 pytestmark = pytest.mark.gpu
 
-S, START = 3200, 5
+S, START = 4200, 5
+LATE = [(1, 600), (1, 4199), (16, 3000), (33, 700), (65, 1983), (128, 2900), (129, 4031), (384, 2690), (500, 3700)]
 COUNTS = [1, 16, 17, 63, 64, 65, 127, 128, 129, 192, 257, 384, 385, 513, 641, 700, 900, 1025, 1281, 2049, 3001]
 
 
@@ -46,11 +50,11 @@ def layer():
             "rows": mk_lib.weights_struct(packed, tiled=False), "ids": ids, "kv": kv}
 
 
-def reference(layer, n, dt):
-    """Hidden state, K and V rows of n tokens at START: bf16 rounding at the
+def reference(layer, n, start, dt):
+    """Hidden state, K and V rows of n tokens at row start: bf16 rounding at the
     kernel's points for dt float32, none for float64."""
     r = (lambda t: t.bfloat16().to(dt)) if dt == torch.float32 else (lambda t: t)
-    sd, rope = layer["sd"], layer["packed"]["rope"][START:START + n].to(dt)
+    sd, rope = layer["sd"], layer["packed"]["rope"][start:start + n].to(dt)
     w = lambda name: sd["layers.0." + name + ".weight"].to(dt).t()
     norm = lambda t: r(t * torch.rsqrt(t.square().mean(-1, keepdim=True) + 1e-5))
 
@@ -64,9 +68,9 @@ def reference(layer, n, dt):
     q = rot(r(x @ w("self_attn.q_proj")).view(n, 32, 64))
     k = rot(r(x @ w("self_attn.k_proj")).view(n, 8, 64))
     v = r(x @ w("self_attn.v_proj")).view(n, 8, 64)
-    keys = torch.cat([layer["kv"][0, :, :START].to(dt), k.transpose(0, 1)], 1)      # [8, START + n, 64]
-    vals = torch.cat([layer["kv"][1, :, :START].to(dt), v.transpose(0, 1)], 1)
-    mask = torch.arange(START + n, device="cuda")[None] > START + torch.arange(n, device="cuda")[:, None]
+    keys = torch.cat([layer["kv"][0, :, :start].to(dt), k.transpose(0, 1)], 1)      # [8, start + n, 64]
+    vals = torch.cat([layer["kv"][1, :, :start].to(dt), v.transpose(0, 1)], 1)
+    mask = torch.arange(start + n, device="cuda")[None] > start + torch.arange(n, device="cuda")[:, None]
     att = torch.empty(n, 32, 64, dtype=dt, device="cuda")
     for hd in range(32):
         s = (q[:, hd] @ keys[hd // 4].t().contiguous() / math.sqrt(64)).masked_fill(mask, float("-inf"))
@@ -79,28 +83,28 @@ def reference(layer, n, dt):
     return r(h1 + r(act @ w("mlp.down_proj"))), k, v
 
 
-def run(layer, n, weights):
+def run(layer, n, start, weights):
     import mk_lib
     kv = layer["kv"].clone()
     out = torch.empty(n, 2048, dtype=torch.bfloat16, device="cuda")
-    mk_lib.prefill(weights, layer["ids"][:n].contiguous(), [kv[0]], [kv[1]], START, mk_lib.prefill_workspace(n, "cuda"),
+    mk_lib.prefill(weights, layer["ids"][:n].contiguous(), [kv[0]], [kv[1]], start, mk_lib.prefill_workspace(n, "cuda"),
                    hidden_out=out)
     torch.cuda.synchronize()
     return out, kv
 
 
-@pytest.mark.parametrize("n", COUNTS)
-def test_layer_at_row_count(layer, n):
-    out, kv = run(layer, n, layer["tiled"])
-    again, kv2 = run(layer, n, layer["rows"])
+@pytest.mark.parametrize("n,start", [(n, START) for n in COUNTS] + LATE)
+def test_layer_at_row_count(layer, n, start):
+    out, kv = run(layer, n, start, layer["tiled"])
+    again, kv2 = run(layer, n, start, layer["rows"])
     assert torch.equal(out.view(torch.int16), again.view(torch.int16))
     assert torch.equal(kv.view(torch.int16), kv2.view(torch.int16))
-    rounded, exact = reference(layer, n, torch.float32), reference(layer, n, torch.float64)
-    rows = slice(START, START + n)
+    rounded, exact = reference(layer, n, start, torch.float32), reference(layer, n, start, torch.float64)
+    rows = slice(start, start + n)
     got = (out, kv[0, :, rows].transpose(0, 1), kv[1, :, rows].transpose(0, 1))
     rms = lambda t: t.double().square().mean().sqrt().item()
     ratios = [rms(g.double() - e) / rms(f.double() - e) for g, f, e in zip(got, rounded, exact)]
-    say(f"[prefill gemm] {n} tokens: departure from exact over the rounded reference's: "
+    say(f"[prefill gemm] {n} tokens at {start}: departure from exact over the rounded reference's: "
         + ", ".join(f"{x:.3f}" for x in ratios))
     assert max(ratios) <= 1.5, ratios
     rest = torch.ones(S, dtype=torch.bool, device="cuda")
