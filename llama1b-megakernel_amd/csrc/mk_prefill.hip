@@ -58,7 +58,7 @@ struct GemmArgs {
   int tiled;
   int M, N, K;
   int mt;                // row tiles
-  int splits;            // EPI_PART: the K range is cut into `splits` parts (blockIdx.y)
+  int splits;            // EPI_PART: the K range is cut into `splits` parts
   const uint16_t* res;   // EPI_RES: residual, row-major [M][N]
   uint16_t* out;         // EPI_RES: row-major [M][N]; EPI_SWIGLU: A-tile order [M16][N/2]; EPI_QKV: q [M][2048]
   float* part;           // EPI_PART: fp32 [splits][M][N]
@@ -113,16 +113,17 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) pf_gemm(GemmArgs g) {
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;   // (uniform: LDS copy bases)
   // Workgroup w runs on XCD w % 8: each XCD gets a contiguous range of tiles,
   // rows first, so the workgroups that share weight columns share its L2.
-  const int nt = g.N / (16 * BB), total = g.mt * nt;
+  const int nt = g.N / (16 * BB), tiles = g.mt * nt, total = EPI == EPI_PART ? tiles * g.splits : tiles;
   const int xcd = blockIdx.x & 7, q8 = total >> 3, r8 = total & 7;
-  const int tile = xcd * q8 + min(xcd, r8) + ((int)blockIdx.x >> 3);
+  const int item = xcd * q8 + min(xcd, r8) + ((int)blockIdx.x >> 3);
+  const int split = EPI == EPI_PART ? item / tiles : 0, tile = EPI == EPI_PART ? item - split * tiles : item;
   const int tm = tile % g.mt, tn = tile / g.mt;
   const int m16 = (g.M + 15) / 16, kb = g.K / 32;
   const rsrc_t ra = make_rsrc(g.a, (size_t)m16 * 16 * g.K * 2);
   const rsrc_t rb = make_rsrc(g.b, (size_t)g.N * g.K * 2);
-  // the k-steps of this workgroup: all of K, or part blockIdx.y of `splits` (an even number)
+  // the k-steps of this workgroup: all of K, or one of `splits` parts (an even number)
   const int kn = EPI == EPI_PART ? kb / g.splits : kb;
-  const int k0 = EPI == EPI_PART ? (int)blockIdx.y * kn : 0, ke = k0 + kn;
+  const int k0 = split * kn, ke = k0 + kn;
   // this wave's blocks of a k-step: wave * CPW + u of the A blocks, then the B blocks
   const uint32_t bstep = g.tiled ? 1024u : 64u;
   const uint32_t arow = (uint32_t)(lane * 16);
@@ -206,7 +207,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) pf_gemm(GemmArgs g) {
       if (m < g.M)
 #pragma unroll
         for (int j = 0; j < NI; ++j)
-          *reinterpret_cast<f32x4*>(g.part + ((size_t)blockIdx.y * g.M + m) * g.N + n0 + 16 * j + 4 * lq) = acc[i][j];
+          *reinterpret_cast<f32x4*>(g.part + ((size_t)split * g.M + m) * g.N + n0 + 16 * j + 4 * lq) = acc[i][j];
     }
     return;
   }
@@ -720,7 +721,7 @@ constexpr int TILES_RES = 4, TILES_PART = 3, TILES_ALL = sizeof(TILES) / sizeof(
 
 template <int EPI, int MI, int NI, int WM, int WN, int NS>
 void gemm_launch(const GemmArgs& g, const GemmTile& t, hipStream_t st) {
-  hipLaunchKernelGGL((pf_gemm<EPI, MI, NI, WM, WN, NS>), dim3(g.mt * (g.N / t.tn), g.splits), dim3(64 * WM * WN), 0, st,
+  hipLaunchKernelGGL((pf_gemm<EPI, MI, NI, WM, WN, NS>), dim3(g.mt * (g.N / t.tn) * g.splits), dim3(64 * WM * WN), 0, st,
                      g);
 }
 template <int EPI>
@@ -758,10 +759,10 @@ float gemm_us(const GemmTile& t, int M, int N, int K, int splits, float tail) {
   const float us = t.fixed + rounds * (t.round + t.kstep * (float)(K / 32 / splits));
   return splits == 1 ? us : us + tail + (float)splits * (float)M * (float)N * 4.f / 7e6f;
 }
-GemmPlan gemm_plan(int M, int N, int K, int tiles, bool split, float tail) {
+GemmPlan gemm_plan(int M, int N, int K, int tiles, size_t part_bytes, float tail) {
   GemmPlan best = {0, 1};
   const int most = (M + 127) / 128 * 128, Ms = most <= 128 ? 64 : most;
-  for (int sp = 2; split && sp <= 16 && (size_t)sp * most * N * 4 <= PART_BYTES; sp *= 2) {
+  for (int sp = 2; sp <= 16 && (size_t)sp * most * N * 4 <= part_bytes; sp *= 2) {
     auto least = [&](int s) {
       const int n = s > 1 ? TILES_PART : tiles;
       float us = gemm_us(TILES[0], Ms, N, K, s, tail);
@@ -802,19 +803,19 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
   uint8_t* base = static_cast<uint8_t*>(a->workspace);
   uint16_t* x = reinterpret_cast<uint16_t*>(base);
   uint16_t* h1 = x + c16 * H;
-  uint16_t* q = h1 + c16 * H;
-  uint16_t* xn = q + c16 * H;
-  uint16_t* att = xn + c16 * H;
-  uint16_t* act = att + c16 * H;
-  float* part = reinterpret_cast<float*>(act + c16 * INTER);
+  uint16_t* xn = h1 + c16 * H;
+  uint16_t* act = xn + c16 * H;
+  uint16_t* att = act + c16 * INTER;
+  uint16_t* q = att + c16 * H;
+  float* part = reinterpret_cast<float*>(q + c16 * H);
   const int L = a->n_layers, l0 = a->first_layer;
   // An N = 2048 projection (O: K = 2048, down: K = 8192) of T tokens with the
   // residual add, followed by the RMSNorm of its output into xn if `norm`:
   // as one GEMM with the add in its epilogue plus pf_norm, or, where few tiles
   // would leave the device idle, split over K into fp32 partials that
   // pf_reduce_norm sums (in split order), adds and normalises.
-  auto res_gemm = [&](GemmArgs g, const uint16_t* res, uint16_t* out, bool norm, int T) {
-    const GemmPlan pl = gemm_plan(T, g.N, g.K, TILES_RES, true, -0.5f);
+  auto res_gemm = [&](GemmArgs g, const uint16_t* res, uint16_t* out, bool norm, int T, float* parts, size_t part_bytes) {
+    const GemmPlan pl = gemm_plan(T, g.N, g.K, TILES_RES, part_bytes, -0.5f);
     g.splits = pl.splits;
     if (pl.splits == 1) {
       g.res = res;
@@ -824,14 +825,14 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
         hipLaunchKernelGGL(pf_norm, dim3((unsigned)((T + NWAVE - 1) / NWAVE)), dim3(NT), 0, st, (const uint16_t*)out,
                            (const int32_t*)nullptr, (const uint16_t*)nullptr, (uint16_t*)nullptr, xn, T);
     } else {
-      g.part = part;
+      g.part = parts;
       gemm_run<EPI_PART>(g, pl.tile, st);
       uint16_t* xn_out = norm ? xn : nullptr;
       switch (pl.splits) {   // gemm_plan gives 2, 4, 8 or 16
-        case 2: hipLaunchKernelGGL(pf_reduce_norm<2>, dim3(T), dim3(NT), 0, st, (const float*)part, res, out, xn_out, T); break;
-        case 4: hipLaunchKernelGGL(pf_reduce_norm<4>, dim3(T), dim3(NT), 0, st, (const float*)part, res, out, xn_out, T); break;
-        case 8: hipLaunchKernelGGL(pf_reduce_norm<8>, dim3(T), dim3(NT), 0, st, (const float*)part, res, out, xn_out, T); break;
-        default: hipLaunchKernelGGL(pf_reduce_norm<16>, dim3(T), dim3(NT), 0, st, (const float*)part, res, out, xn_out, T); break;
+        case 2: hipLaunchKernelGGL(pf_reduce_norm<2>, dim3(T), dim3(NT), 0, st, (const float*)parts, res, out, xn_out, T); break;
+        case 4: hipLaunchKernelGGL(pf_reduce_norm<4>, dim3(T), dim3(NT), 0, st, (const float*)parts, res, out, xn_out, T); break;
+        case 8: hipLaunchKernelGGL(pf_reduce_norm<8>, dim3(T), dim3(NT), 0, st, (const float*)parts, res, out, xn_out, T); break;
+        default: hipLaunchKernelGGL(pf_reduce_norm<16>, dim3(T), dim3(NT), 0, st, (const float*)parts, res, out, xn_out, T); break;
       }
     }
   };
@@ -863,7 +864,7 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
       g.out = q;
       g.kc = kc;
       g.vc = vc;
-      const GemmPlan qp = gemm_plan(T, QKV_ROWS, H, TILES_ALL, true, 4.5f);
+      const GemmPlan qp = gemm_plan(T, QKV_ROWS, H, TILES_ALL, PART_BYTES, 4.5f);
       g.splits = qp.splits;
       if (qp.splits == 1) {
         gemm_run<EPI_QKV>(g, qp.tile, st);
@@ -897,7 +898,7 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
       g.N = H;
       g.K = H;
       g.kc = g.vc = nullptr;
-      res_gemm(g, x, h1, true, T);
+      res_gemm(g, x, h1, true, T, part, PART_BYTES);
       // gate/up + SwiGLU -> act
       g.a = xn;
       g.b = Wgu + (size_t)l * 2 * INTER * H;
@@ -905,15 +906,18 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
       g.K = H;
       g.out = act;
       g.splits = 1;
-      gemm_run<EPI_SWIGLU>(g, gemm_plan(T, g.N, g.K, TILES_ALL, false, 0.f).tile, st);
+      gemm_run<EPI_SWIGLU>(g, gemm_plan(T, g.N, g.K, TILES_ALL, 0, 0.f).tile, st);
       // down projection + residual -> x (the next layer's input) and its RMSNorm -> xn,
       // or the caller's hidden state after the last layer
       g.a = act;
       g.b = Wd + (size_t)l * H * INTER;
       g.N = H;
       g.K = INTER;
-      if (li + 1 < L) res_gemm(g, h1, x, true, T);
-      else res_gemm(g, h1, static_cast<uint16_t*>(a->hidden_out) + (size_t)c0 * H, false, T);
+      // (att and q hold nothing any more and lie before `part`)
+      float* down_part = reinterpret_cast<float*>(att);
+      const size_t down_bytes = PART_BYTES + (size_t)T * H * 2 * 2;
+      if (li + 1 < L) res_gemm(g, h1, x, true, T, down_part, down_bytes);
+      else res_gemm(g, h1, static_cast<uint16_t*>(a->hidden_out) + (size_t)c0 * H, false, T, down_part, down_bytes);
     }
   }
   return hipGetLastError();
