@@ -316,14 +316,14 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) pf_gemm(GemmArgs g) {
 // The split-K tail of the O and down projections (N = 2048), one workgroup per
 // token row t, 8 columns per thread: v = the sum of the SPLITS fp32 partials in
 // split order, out = bf16(res + bf16(v)) (row-major), and, if xn is given, the
-// next RMSNorm of out into xn (A-tile order), as pf_norm computes it. Latency
+// next RMSNorm of out into xn (A-tile order), with pf_norm's bits. Latency
 // bounds it: every load of the row is in flight at once (33 tokens of 16 splits
 // on one wave per row, four rounds of loads: 9.4 us).
 template <int SPLITS>
 __global__ void __launch_bounds__(NT) pf_reduce_norm(const float* part, const uint16_t* res, uint16_t* out,
                                                      uint16_t* xn, int T) {
   static_assert(H == 8 * NT, "8 columns per thread");
-  __shared__ float sums[NWAVE];
+  __shared__ u32x4 row[NT];
   const int t = blockIdx.x, c = (int)threadIdx.x * 8;
   float4 pv[SPLITS][2];
 #pragma unroll
@@ -346,13 +346,18 @@ __global__ void __launch_bounds__(NT) pf_reduce_norm(const float* part, const ui
   for (int e = 0; e < 4; ++e) o[e] = pack_bf2(bf_lo(rw[e]) + rbf(v[2 * e]), bf_hi(rw[e]) + rbf(v[2 * e + 1]));
   *reinterpret_cast<u32x4*>(out + (size_t)t * H + c) = u32x4{o[0], o[1], o[2], o[3]};
   if (!xn) return;
+  // every wave sums the whole row's squares, in rmsnorm2048's order
+  row[threadIdx.x] = u32x4{o[0], o[1], o[2], o[3]};
+  __syncthreads();
   float ss = 0.f;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) ss = fmaf(bf_hi(o[e]), bf_hi(o[e]), fmaf(bf_lo(o[e]), bf_lo(o[e]), ss));
-  ss = wave_sum(ss);
-  if (lane_id() == 0) sums[wave_id()] = ss;
-  __syncthreads();
-  const float inv = rsqrtf(((sums[0] + sums[1]) + (sums[2] + sums[3])) * (1.0f / H) + EPS);
+  for (int i = 0; i < H / 512; ++i) {
+    const u32x4 x = row[64 * i + lane_id()];
+    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss = fmaf(bf_hi(w[e]), bf_hi(w[e]), fmaf(bf_lo(w[e]), bf_lo(w[e]), ss));
+  }
+  const float inv = rsqrtf(wave_sum(ss) * (1.0f / H) + EPS);
 #pragma unroll
   for (int e = 0; e < 4; ++e) o[e] = cvt_bf2(bf_lo(o[e]) * inv, bf_hi(o[e]) * inv);
   *reinterpret_cast<u32x4*>(xn + a_tile_off(t, c, H / 32)) = u32x4{o[0], o[1], o[2], o[3]};
@@ -441,6 +446,7 @@ struct AttnArgs {
   int nsplit;
 };
 
+constexpr int EARLY = 128;            // prompts within so many rows: fixed order of all sums (attn_run)
 constexpr int KB = 64;                // keys per step
 constexpr int VT_LD = KB + 8;         // bf16 per row (one dim) of the transposed V tile: 144 bytes
 constexpr int ANS = 3;                // steps of K and V in LDS
@@ -473,7 +479,10 @@ struct AttnTile {
 // Measured against 16-token workgroups with 32-key steps, one step ahead, and V
 // transposed by 2-byte stores: 3001 tokens 112 -> 69 us, 1100 tokens 28.8 -> 23.
 // Three and four tiles per wave are slower than two (84 and 94 us at 3001).
-template <int NTL, bool SPLIT>
+//
+// HALVES: the running maximum moves every 32 keys, and scores are exponentiated
+// as they are: the outputs of 32-key steps bit for bit (attn_run).
+template <int NTL, bool SPLIT, bool HALVES>
 __global__ void __launch_bounds__(NT, NTL > 2 ? 2 : 3) pf_attn(AttnArgs a) {
   __shared__ AttnTile L[ANS];
   const int h = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), tid_ = threadIdx.x, lane = tid_ & 63;
@@ -537,7 +546,49 @@ __global__ void __launch_bounds__(NT, NTL > 2 ? 2 : 3) pf_attn(AttnArgs a) {
 #pragma unroll
     for (int d = 0; d < 4; ++d) acc[j][d] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
+  // the 32 keys hf of a step at a time
+  auto compute_half = [&](int k0, int hf, const AttnTile& cur) {
+    const int lim = a.p0 + min(t0 + col, a.T - 1);   // (padding tokens: any finite row)
+    float s[2][4], mb = -INFINITY;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      const u32x4 ka = cur.k[4 * hf + 2 * kt][lane], kb = cur.k[4 * hf + 2 * kt + 1][lane];
+      const f32x4 v = mfma16(kb, qv[0][1], mfma16(ka, qv[0][0], f32x4{0.f, 0.f, 0.f, 0.f}));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[kt][i] = k0 + 32 * hf + 16 * kt + 4 * q4 + i <= lim ? v[i] * SM_SCALE : -INFINITY;
+        mb = fmaxf(mb, s[kt][i]);
+      }
+    }
+    const float m_new = fmaxf(m_run[0], max_xor32(max_xor16(mb)));   // finite: every token sees key 0
+    const float alpha = __expf(m_run[0] - m_new);
+    m_run[0] = m_new;
+    float p[2][4], ps = 0.f;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        p[kt][i] = __expf(s[kt][i] - m_new);
+        ps += p[kt][i];
+      }
+    l_run[0] = l_run[0] * alpha + ps;
+    const u32x4 pb = {cvt_bf2(p[0][0], p[0][1]), cvt_bf2(p[0][2], p[0][3]), cvt_bf2(p[1][0], p[1][1]),
+                      cvt_bf2(p[1][2], p[1][3])};
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const u32x4 vo = *reinterpret_cast<const u32x4*>(&cur.vt[16 * d + col][32 * hf + 8 * q4]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[0][d][i] *= alpha;
+      acc[0][d] = mfma16(vo, pb, acc[0][d]);
+    }
+  };
   auto compute = [&](int k0, const AttnTile& cur) {
+    if constexpr (HALVES) {
+      static_assert(NTL == 1 && !SPLIT, "one tile, all keys");
+      compute_half(k0, 0, cur);
+      compute_half(k0, 1, cur);
+      return;
+    }
     // S^T: keys 16 kt + 4 q4 + i of the step, this lane's token of each tile
     f32x4 s[NTL][4];
 #pragma unroll
@@ -670,10 +721,10 @@ __global__ void __launch_bounds__(NT) pf_attn_merge(AttnArgs a, int tokens_per_w
       uint2{pack_bf2(o[0] * inv, o[1] * inv), pack_bf2(o[2] * inv, o[3] * inv)};
 }
 
-template <int NTL, bool SPLIT>
+template <int NTL, bool SPLIT, bool HALVES = false>
 void attn_launch(const AttnArgs& a, hipStream_t st) {
   const int nblk = (a.T + 16 * NTL - 1) / (16 * NTL);
-  hipLaunchKernelGGL((pf_attn<NTL, SPLIT>), dim3(nblk * NKV * (SPLIT ? a.nsplit : 1)), dim3(NT), 0, st, a);
+  hipLaunchKernelGGL((pf_attn<NTL, SPLIT, HALVES>), dim3(nblk * NKV * (SPLIT ? a.nsplit : 1)), dim3(NT), 0, st, a);
   if (SPLIT) hipLaunchKernelGGL(pf_attn_merge, dim3((a.T * NQ + NT / 16 - 1) / (NT / 16)), dim3(NT), 0, st, a, 16 * NTL);
 }
 // Tiles of 16 tokens up to 2048 tokens, of 32 above (one 16-token tile per wave
@@ -683,7 +734,14 @@ void attn_launch(const AttnArgs& a, hipStream_t st) {
 // takes one workgroup 0.85 us, the parts and the merge 5 us and what they move
 // (33 tokens at 4000 rows: 55 us whole, 17.5 in 8 parts; at 700 rows 13.6 and
 // 11.0). Splits begin at multiples of 64 keys of the cache.
+//
+// Prompts within the first EARLY rows take the running maximum over 32 keys
+// (HALVES) and fixed K splits (gemm_plan): the bits of the 32-key kernel and its
+// splits, whatever a call's number of tokens. One layer (before: that kernel, its GEMMs):
+// 20 tokens 73.6 -> 45.8 us, 64 83.7 -> 53.6; 128 tokens take 72 us, about 65 with
+// the splits of later rows (16.8 MB of partials instead of 8.4).
 void attn_run(AttnArgs a, hipStream_t st) {
+  if (a.p0 + a.T <= EARLY) return attn_launch<1, false, true>(a, st);
   const int n_keys = a.p0 + a.T, wgs = (a.T + 15) / 16 * NKV;
   const int most = (int)(PART_BYTES / ((size_t)NQ * (HD + 2) * 4)) / a.T;   // splits whose parts fit
   const int ns = min(min(8, 3 * 256 / wgs), most);
@@ -749,7 +807,9 @@ void gemm_run(GemmArgs g, int tile, hipStream_t st) {
 // is the same whatever the tile (its k-steps are summed in order) but not
 // whatever the split, so the splits are those of M rounded up to 128 tokens
 // (of 64 for the first 128, where short turns lie): a prompt of up to 128
-// tokens gives the same bits in any chunks.
+// tokens gives the same bits in any chunks. Prompts within the first EARLY rows
+// have fixed splits (attn_run), EARLY_QKV and EARLY_RES.
+constexpr int EARLY_QKV = 8, EARLY_RES = 16;
 struct GemmPlan {
   int tile, splits;
 };
@@ -759,10 +819,10 @@ float gemm_us(const GemmTile& t, int M, int N, int K, int splits, float tail) {
   const float us = t.fixed + rounds * (t.round + t.kstep * (float)(K / 32 / splits));
   return splits == 1 ? us : us + tail + (float)splits * (float)M * (float)N * 4.f / 7e6f;
 }
-GemmPlan gemm_plan(int M, int N, int K, int tiles, size_t part_bytes, float tail) {
-  GemmPlan best = {0, 1};
+GemmPlan gemm_plan(int M, int N, int K, int tiles, size_t part_bytes, float tail, int fixed = 0) {
+  GemmPlan best = {0, fixed ? fixed : 1};
   const int most = (M + 127) / 128 * 128, Ms = most <= 128 ? 64 : most;
-  for (int sp = 2; sp <= 16 && (size_t)sp * most * N * 4 <= part_bytes; sp *= 2) {
+  for (int sp = 2; !fixed && sp <= 16 && (size_t)sp * most * N * 4 <= part_bytes; sp *= 2) {
     auto least = [&](int s) {
       const int n = s > 1 ? TILES_PART : tiles;
       float us = gemm_us(TILES[0], Ms, N, K, s, tail);
@@ -814,8 +874,9 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
   // as one GEMM with the add in its epilogue plus pf_norm, or, where few tiles
   // would leave the device idle, split over K into fp32 partials that
   // pf_reduce_norm sums (in split order), adds and normalises.
-  auto res_gemm = [&](GemmArgs g, const uint16_t* res, uint16_t* out, bool norm, int T, float* parts, size_t part_bytes) {
-    const GemmPlan pl = gemm_plan(T, g.N, g.K, TILES_RES, part_bytes, -0.5f);
+  auto res_gemm = [&](GemmArgs g, const uint16_t* res, uint16_t* out, bool norm, int T, float* parts, size_t part_bytes,
+                      bool early) {
+    const GemmPlan pl = gemm_plan(T, g.N, g.K, TILES_RES, part_bytes, -0.5f, early ? EARLY_RES : 0);
     g.splits = pl.splits;
     if (pl.splits == 1) {
       g.res = res;
@@ -841,6 +902,7 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
   // only its QKV GEMM unless the hidden state is asked for.
   for (int c0 = 0; c0 < a->n_tokens; c0 += cap) {
     const int T = min(cap, a->n_tokens - c0), p0 = a->start_pos + c0;
+    const bool early = p0 + T <= EARLY;
     hipLaunchKernelGGL(pf_norm, dim3((T + NWAVE - 1) / NWAVE), dim3(NT), 0, st, (const uint16_t*)nullptr,
                        a->tokens + c0, static_cast<const uint16_t*>(w->embed), x, xn, T);
     for (int li = 0; li < L; ++li) {
@@ -864,7 +926,7 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
       g.out = q;
       g.kc = kc;
       g.vc = vc;
-      const GemmPlan qp = gemm_plan(T, QKV_ROWS, H, TILES_ALL, PART_BYTES, 4.5f);
+      const GemmPlan qp = gemm_plan(T, QKV_ROWS, H, TILES_ALL, PART_BYTES, 4.5f, early ? EARLY_QKV : 0);
       g.splits = qp.splits;
       if (qp.splits == 1) {
         gemm_run<EPI_QKV>(g, qp.tile, st);
@@ -898,7 +960,7 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
       g.N = H;
       g.K = H;
       g.kc = g.vc = nullptr;
-      res_gemm(g, x, h1, true, T, part, PART_BYTES);
+      res_gemm(g, x, h1, true, T, part, PART_BYTES, early);
       // gate/up + SwiGLU -> act
       g.a = xn;
       g.b = Wgu + (size_t)l * 2 * INTER * H;
@@ -916,8 +978,8 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
       // (att and q hold nothing any more and lie before `part`)
       float* down_part = reinterpret_cast<float*>(att);
       const size_t down_bytes = PART_BYTES + (size_t)T * H * 2 * 2;
-      if (li + 1 < L) res_gemm(g, h1, x, true, T, down_part, down_bytes);
-      else res_gemm(g, h1, static_cast<uint16_t*>(a->hidden_out) + (size_t)c0 * H, false, T, down_part, down_bytes);
+      if (li + 1 < L) res_gemm(g, h1, x, true, T, down_part, down_bytes, early);
+      else res_gemm(g, h1, static_cast<uint16_t*>(a->hidden_out) + (size_t)c0 * H, false, T, down_part, down_bytes, early);
     }
   }
   return hipGetLastError();

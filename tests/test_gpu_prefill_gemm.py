@@ -28,7 +28,7 @@ from gpu_common import need_gpu, say
 pytestmark = pytest.mark.gpu
 
 S, START = 4200, 5
-LATE = [(1, 600), (1, 4199), (16, 3000), (33, 700), (65, 1983), (128, 2900), (129, 4031), (384, 2690), (500, 3700)]
+LATE = [(64, 64), (123, 5), (124, 5), (128, 0), (128, 1), (1, 600), (1, 4199), (16, 3000), (33, 700), (65, 1983), (128, 2900), (129, 4031), (384, 2690), (500, 3700)]
 COUNTS = [1, 16, 17, 63, 64, 65, 127, 128, 129, 192, 257, 384, 385, 513, 641, 700, 900, 1025, 1281, 2049, 3001]
 
 
@@ -110,3 +110,23 @@ def test_layer_at_row_count(layer, n, start):
     rest = torch.ones(S, dtype=torch.bool, device="cuda")
     rest[rows] = False
     assert torch.equal(kv[:, :, rest].view(torch.int16), layer["kv"][:, :, rest].view(torch.int16))
+
+
+@pytest.mark.parametrize("n", [2, 33, 64, 65, 128])
+@pytest.mark.parametrize("cut", [1, 32, 63, 64])
+def test_prompt_within_128_rows_in_any_chunks(layer, n, cut):
+    """Whole or cut in two, a prompt within the first 128 rows gives the same
+    bits: its K splits and the attention's 32-key steps do not depend on how
+    many tokens a call has."""
+    import mk_lib
+    if cut >= n:
+        pytest.skip("nothing to cut")
+    out, kv = run(layer, n, 0, layer["tiled"])
+    kv2 = layer["kv"].clone()
+    out2 = torch.empty_like(out)
+    ws = mk_lib.prefill_workspace(n, "cuda")
+    for a, b in ((0, cut), (cut, n)):
+        mk_lib.prefill(layer["tiled"], layer["ids"][a:b].clone(), [kv2[0]], [kv2[1]], a, ws, hidden_out=out2[a:b])
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), out2.view(torch.int16))
+    assert torch.equal(kv.view(torch.int16), kv2.view(torch.int16))
