@@ -39,6 +39,8 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <type_traits>
+
 #include "mk.h"
 #include "mk_common.h"
 #include "mk_prefill.h"
@@ -121,9 +123,9 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) pf_gemm(GemmArgs g) {
   const int m16 = (g.M + 15) / 16, kb = g.K / 32;
   const rsrc_t ra = make_rsrc(g.a, (size_t)m16 * 16 * g.K * 2);
   const rsrc_t rb = make_rsrc(g.b, (size_t)g.N * g.K * 2);
-  // the k-steps of this workgroup: all of K, or one of `splits` parts (an even number)
-  const int kn = EPI == EPI_PART ? kb / g.splits : kb;
-  const int k0 = split * kn, ke = k0 + kn;
+  // the k-steps of this workgroup: all of K, or one of `splits` parts (even numbers, as equal as they can be)
+  const int k0 = EPI == EPI_PART ? kb / 2 * split / g.splits * 2 : 0;
+  const int ke = EPI == EPI_PART ? kb / 2 * (split + 1) / g.splits * 2 : kb;
   // this wave's blocks of a k-step: wave * CPW + u of the A blocks, then the B blocks
   const uint32_t bstep = g.tiled ? 1024u : 64u;
   const uint32_t arow = (uint32_t)(lane * 16);
@@ -813,16 +815,34 @@ constexpr int EARLY_QKV = 8, EARLY_RES = 16;
 struct GemmPlan {
   int tile, splits;
 };
+// The splits the tails are built for; f(std::integral_constant<int, splits>).
+// (3 and 5 fill the device where 2 and 4 leave a quarter of it idle and the
+// partials of 8 do not fit: the down projection of 383 tokens on 240 workgroups
+// instead of 192 takes 20.4 us instead of 23.1, its tail 6.0 instead of 5.8; the
+// parts of K then differ by one pair of k-steps.)
+constexpr int SPLITS[] = {2, 3, 4, 5, 8, 16};
+template <class F>
+void with_splits(int splits, F&& f) {
+  switch (splits) {
+    case 2: return f(std::integral_constant<int, 2>{});
+    case 3: return f(std::integral_constant<int, 3>{});
+    case 4: return f(std::integral_constant<int, 4>{});
+    case 5: return f(std::integral_constant<int, 5>{});
+    case 8: return f(std::integral_constant<int, 8>{});
+    case 16: return f(std::integral_constant<int, 16>{});
+  }
+}
 float gemm_us(const GemmTile& t, int M, int N, int K, int splits, float tail) {
   const int wg = (M + t.tm - 1) / t.tm * (N / t.tn) * splits;
   const float rounds = t.tm == 64 ? fmaxf(1.f, (float)wg / 256.f) : (float)((wg + 255) / 256);
-  const float us = t.fixed + rounds * (t.round + t.kstep * (float)(K / 32 / splits));
+  const float us = t.fixed + rounds * (t.round + t.kstep * (float)((K / 64 + splits - 1) / splits * 2));
   return splits == 1 ? us : us + tail + (float)splits * (float)M * (float)N * 4.f / 7e6f;
 }
 GemmPlan gemm_plan(int M, int N, int K, int tiles, size_t part_bytes, float tail, int fixed = 0) {
   GemmPlan best = {0, fixed ? fixed : 1};
   const int most = (M + 127) / 128 * 128, Ms = most <= 128 ? 64 : most;
-  for (int sp = 2; !fixed && sp <= 16 && (size_t)sp * most * N * 4 <= part_bytes; sp *= 2) {
+  for (int sp : SPLITS) {
+    if (fixed || (size_t)sp * most * N * 4 > part_bytes) break;
     auto least = [&](int s) {
       const int n = s > 1 ? TILES_PART : tiles;
       float us = gemm_us(TILES[0], Ms, N, K, s, tail);
@@ -889,12 +909,9 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
       g.part = parts;
       gemm_run<EPI_PART>(g, pl.tile, st);
       uint16_t* xn_out = norm ? xn : nullptr;
-      switch (pl.splits) {   // gemm_plan gives 2, 4, 8 or 16
-        case 2: hipLaunchKernelGGL(pf_reduce_norm<2>, dim3(T), dim3(NT), 0, st, (const float*)parts, res, out, xn_out, T); break;
-        case 4: hipLaunchKernelGGL(pf_reduce_norm<4>, dim3(T), dim3(NT), 0, st, (const float*)parts, res, out, xn_out, T); break;
-        case 8: hipLaunchKernelGGL(pf_reduce_norm<8>, dim3(T), dim3(NT), 0, st, (const float*)parts, res, out, xn_out, T); break;
-        default: hipLaunchKernelGGL(pf_reduce_norm<16>, dim3(T), dim3(NT), 0, st, (const float*)parts, res, out, xn_out, T); break;
-      }
+      with_splits(pl.splits, [&](auto n) {
+        hipLaunchKernelGGL(pf_reduce_norm<n.value>, dim3(T), dim3(NT), 0, st, (const float*)parts, res, out, xn_out, T);
+      });
     }
   };
   // Every chunk starts again from the embeddings of its own tokens; the rows
@@ -935,12 +952,10 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
         gemm_run<EPI_PART>(g, qp.tile, st);
         const uint16_t* rope = static_cast<const uint16_t*>(w->rope);
         const dim3 fg(T, QKV_PAIRS / 2 / NT);
-        switch (qp.splits) {   // gemm_plan gives 2, 4, 8 or 16
-          case 2: hipLaunchKernelGGL(pf_qkv_finish<2>, fg, dim3(NT), 0, st, (const float*)part, rope, q, kc, vc, T, p0, a->s_max); break;
-          case 4: hipLaunchKernelGGL(pf_qkv_finish<4>, fg, dim3(NT), 0, st, (const float*)part, rope, q, kc, vc, T, p0, a->s_max); break;
-          case 8: hipLaunchKernelGGL(pf_qkv_finish<8>, fg, dim3(NT), 0, st, (const float*)part, rope, q, kc, vc, T, p0, a->s_max); break;
-          default: hipLaunchKernelGGL(pf_qkv_finish<16>, fg, dim3(NT), 0, st, (const float*)part, rope, q, kc, vc, T, p0, a->s_max); break;
-        }
+        with_splits(qp.splits, [&](auto n) {
+          hipLaunchKernelGGL(pf_qkv_finish<n.value>, fg, dim3(NT), 0, st, (const float*)part, rope, q, kc, vc, T, p0,
+                             a->s_max);
+        });
         g.splits = 1;
       }
       if (tail) break;   // the last layer's K/V rows are all the caller needs
