@@ -29,11 +29,12 @@
 // partials are summed in a fixed order by pf_reduce_norm (O and down) and
 // pf_qkv_finish (QKV, with RoPE and the scatter).
 //
-// Attention: per (kv head, block of 16 tokens) one workgroup; S^T = K Q^T on
-// the matrix cores (keys on M, the 16 tokens x 4 q heads on N), an online
-// softmax per (token, head) column, and O^T = V^T P^T on the matrix cores with
-// p rounded to bf16 as the reference rounds it (relative to the running
-// maximum). K and V tiles of 32 keys go through LDS (V transposed there).
+// Attention: per (kv head, block of 16 or 32 tokens, range of keys) one
+// workgroup, a q head per wave; S^T = K Q^T on the matrix cores (keys on M, 16
+// tokens on N), an online softmax per column, and O^T = V^T P^T on the matrix
+// cores with p rounded to bf16 as the reference rounds it (relative to the
+// running maximum). K and V go through LDS in steps of 64 keys (V transposed
+// there); where the keys are split, pf_attn_merge combines the parts.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
