@@ -24,10 +24,11 @@
 // activations are kept in A-tile order (the producing kernel writes them so)
 // and the weights are the MFMA-tiled copies, so each k-step's operands of an
 // output tile are blocks of 1 KiB that go from memory straight into LDS. The
-// tile (64x64 to 256x256) and, for short prompts, a split of K into fp32
-// partials are chosen per projection by estimated time (gemm_plan); the
-// partials are summed in a fixed order by pf_reduce_norm (O and down) and
-// pf_qkv_finish (QKV, with RoPE and the scatter).
+// tile (64x64 to 256x256) and, for few tokens, a split of K into fp32 partials are
+// chosen per projection by estimated time (gemm_tile, gemm_splits; calls of up to
+// 128 tokens have splits of their own, gemm_short); the partials are summed in a
+// fixed order by pf_reduce_norm (O and down) and pf_qkv_finish (QKV, with RoPE and
+// the scatter).
 //
 // Attention: per (kv head, block of 16 or 32 tokens, range of keys) one
 // workgroup, a q head per wave; S^T = K Q^T on the matrix cores (keys on M, 16
@@ -53,7 +54,16 @@ using namespace mk;
 // fp32 partials: a projection's (splits * M * N floats) or the attention's key splits
 constexpr size_t PART_BYTES = (size_t)2048 * H * 4;
 
-enum : int { EPI_QKV = 0, EPI_RES = 1, EPI_SWIGLU = 2, EPI_PART = 3 };
+// Short calls, of up to SHORT_TOKENS tokens, give every token the same bits however
+// a prompt is cut into them, at any row: the order of all its sums follows from its
+// row in the cache alone. The first EARLY_ROWS rows keep the order that short
+// prompts have always had, so their outputs have not changed: K in SHORT_QKV or
+// SHORT_RES parts, the attention's maximum over 32 keys. Later rows take a faster
+// one: half as many parts, each the sum of two, maxima over 64 keys, and the keys
+// split (gemm_short, pf_attn, short_split).
+constexpr int SHORT_TOKENS = 128, EARLY_ROWS = 128;
+
+enum : int { EPI_QKV = 0, EPI_RES = 1, EPI_SWIGLU = 2, EPI_PART = 3, EPI_PAIR = 4 };
 
 struct GemmArgs {
   const uint16_t* a;     // activations, A-tile order [M16][K]
@@ -61,10 +71,10 @@ struct GemmArgs {
   int tiled;
   int M, N, K;
   int mt;                // row tiles
-  int splits;            // EPI_PART: the K range is cut into `splits` parts
+  int splits;            // EPI_PART, EPI_PAIR: the K range is cut into `splits` parts
   const uint16_t* res;   // EPI_RES: residual, row-major [M][N]
   uint16_t* out;         // EPI_RES: row-major [M][N]; EPI_SWIGLU: A-tile order [M16][N/2]; EPI_QKV: q [M][2048]
-  float* part;           // EPI_PART: fp32 [splits][M][N]
+  float* part;           // EPI_PART, EPI_PAIR: fp32 [splits][M][N]
   uint16_t* kc;          // EPI_QKV: the layer's caches, bf16 [8][s_max][64]
   uint16_t* vc;
   const uint16_t* rope;  // bf16 [rows][128]
@@ -92,7 +102,7 @@ __device__ __forceinline__ void wait_copies() {
 // 128x64 halves the copies per MFMA and puts two waves on a SIMD, so that one
 // multiplies while the other waits: 16384 x 2048 weights at 3000 tokens 208 ->
 // 147 us (1370 TFLOP/s). Smaller tiles serve the shapes that would leave the
-// device idle (gemm_plan).
+// device idle (gemm_tile).
 //
 // Operands are 1 KiB blocks (16 rows x 32 columns) copied from memory straight
 // into a ring of NS k-steps in LDS, NS - 1 ahead; each wave reads the next
@@ -107,6 +117,7 @@ __device__ __forceinline__ void wait_copies() {
 // 2-byte stores of the transposed form took 14 us per round of 256x256 tiles.
 template <int EPI, int MI, int NI, int WM, int WN, int NS>
 __global__ void __launch_bounds__(64 * WM * WN, 2) pf_gemm(GemmArgs g) {
+  constexpr bool SPLIT_K = EPI == EPI_PART || EPI == EPI_PAIR;
   constexpr int NW = WM * WN, AB = MI * WM, BB = NI * WN, NB = AB + BB;   // waves; A, B and all blocks of a k-step
   constexpr int CPW = (NB + NW - 1) / NW;                                // copies per wave and k-step
   constexpr bool SPARE = NB % NW != 0;                                   // the last wave's surplus copies
@@ -116,17 +127,18 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) pf_gemm(GemmArgs g) {
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;   // (uniform: LDS copy bases)
   // Workgroup w runs on XCD w % 8: each XCD gets a contiguous range of tiles,
   // rows first, so the workgroups that share weight columns share its L2.
-  const int nt = g.N / (16 * BB), tiles = g.mt * nt, total = EPI == EPI_PART ? tiles * g.splits : tiles;
+  const int nt = g.N / (16 * BB), tiles = g.mt * nt, total = SPLIT_K ? tiles * g.splits : tiles;
   const int xcd = blockIdx.x & 7, q8 = total >> 3, r8 = total & 7;
   const int item = xcd * q8 + min(xcd, r8) + ((int)blockIdx.x >> 3);
-  const int split = EPI == EPI_PART ? item / tiles : 0, tile = EPI == EPI_PART ? item - split * tiles : item;
+  const int split = SPLIT_K ? item / tiles : 0, tile = SPLIT_K ? item - split * tiles : item;
   const int tm = tile % g.mt, tn = tile / g.mt;
   const int m16 = (g.M + 15) / 16, kb = g.K / 32;
   const rsrc_t ra = make_rsrc(g.a, (size_t)m16 * 16 * g.K * 2);
   const rsrc_t rb = make_rsrc(g.b, (size_t)g.N * g.K * 2);
   // the k-steps of this workgroup: all of K, or one of `splits` parts (even numbers, as equal as they can be)
-  const int k0 = EPI == EPI_PART ? kb / 2 * split / g.splits * 2 : 0;
-  const int ke = EPI == EPI_PART ? kb / 2 * (split + 1) / g.splits * 2 : kb;
+  const int k0 = SPLIT_K ? kb / 2 * split / g.splits * 2 : 0;
+  const int ke = SPLIT_K ? kb / 2 * (split + 1) / g.splits * 2 : kb;
+  const int kmid = (k0 + ke) / 4 * 2;   // EPI_PAIR: the second half, summed from zero, begins here
   // this wave's blocks of a k-step: wave * CPW + u of the A blocks, then the B blocks
   const uint32_t bstep = g.tiled ? 1024u : 64u;
   const uint32_t arow = (uint32_t)(lane * 16);
@@ -171,7 +183,18 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) pf_gemm(GemmArgs g) {
   int stg = 0, fill = NS - 1;
   wait_copies<(NS - 2) * CPW, 0>();
   read(0, av[0], bv[0]);
+  f32x4 first[EPI == EPI_PAIR ? MI : 1][EPI == EPI_PAIR ? NI : 1];
   for (int ks = k0; ks < ke; ks += 2) {
+    if constexpr (EPI == EPI_PAIR)
+      if (ks == kmid) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) {
+            first[i][j] = acc[i][j];
+            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+      }
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       // k-step ks + s + 1 is in LDS, and every wave has read the stage refilled
@@ -203,10 +226,13 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) pf_gemm(GemmArgs g) {
   // epilogue: acc[i][j][r] is (row m0(i) + lane%16, column n0 + 16j + 4*(lane/16) + r)
   const int n0 = 16 * (tn * BB + NI * wn), mw = 16 * (tm * AB + MI * wm);
   const int lm = lane & 15, lq = lane >> 4;
-  if constexpr (EPI == EPI_PART) {
+  if constexpr (SPLIT_K) {
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
       const int m = mw + 16 * i + lm;
+      if constexpr (EPI == EPI_PAIR)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) acc[i][j] = first[i][j] + acc[i][j];
       if (m < g.M)
 #pragma unroll
         for (int j = 0; j < NI; ++j)
@@ -316,15 +342,20 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) pf_gemm(GemmArgs g) {
   }
 }
 
+__device__ __forceinline__ float4 sum4(const float4& a, const float4& b) {
+  return float4{a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w};
+}
+
 // The split-K tail of the O and down projections (N = 2048), one workgroup per
 // token row t, 8 columns per thread: v = the sum of the SPLITS fp32 partials in
-// split order, out = bf16(res + bf16(v)) (row-major), and, if xn is given, the
+// split order (MIXED, a short call across EARLY_ROWS: of their pairs' sums from that
+// row on), out = bf16(res + bf16(v)) (row-major), and, if xn is given, the
 // next RMSNorm of out into xn (A-tile order), with pf_norm's bits. Latency
 // bounds it: every load of the row is in flight at once (33 tokens of 16 splits
 // on one wave per row, four rounds of loads: 9.4 us).
-template <int SPLITS>
+template <int SPLITS, bool MIXED>
 __global__ void __launch_bounds__(NT) pf_reduce_norm(const float* part, const uint16_t* res, uint16_t* out,
-                                                     uint16_t* xn, int T) {
+                                                     uint16_t* xn, int T, int p0) {
   static_assert(H == 8 * NT, "8 columns per thread");
   __shared__ u32x4 row[NT];
   const int t = blockIdx.x, c = (int)threadIdx.x * 8;
@@ -337,11 +368,16 @@ __global__ void __launch_bounds__(NT) pf_reduce_norm(const float* part, const ui
   }
   const u32x4 rv = *reinterpret_cast<const u32x4*>(res + (size_t)t * H + c);
   float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  auto add = [&](const float4& a, const float4& b) {
+    v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w;
+    v[4] += b.x; v[5] += b.y; v[6] += b.z; v[7] += b.w;
+  };
+  if (MIXED && p0 + t >= EARLY_ROWS) {
 #pragma unroll
-  for (int sp = 0; sp < SPLITS; ++sp) {
-    const float4 p0 = pv[sp][0], p1 = pv[sp][1];
-    v[0] += p0.x; v[1] += p0.y; v[2] += p0.z; v[3] += p0.w;
-    v[4] += p1.x; v[5] += p1.y; v[6] += p1.z; v[7] += p1.w;
+    for (int sp = 0; sp + 1 < SPLITS; sp += 2) add(sum4(pv[sp][0], pv[sp + 1][0]), sum4(pv[sp][1], pv[sp + 1][1]));
+  } else {
+#pragma unroll
+    for (int sp = 0; sp < SPLITS; ++sp) add(pv[sp][0], pv[sp][1]);
   }
   const uint32_t rw[4] = {rv.x, rv.y, rv.z, rv.w};
   uint32_t o[4];
@@ -366,14 +402,14 @@ __global__ void __launch_bounds__(NT) pf_reduce_norm(const float* part, const ui
   *reinterpret_cast<u32x4*>(xn + a_tile_off(t, c, H / 32)) = u32x4{o[0], o[1], o[2], o[3]};
 }
 
-// The split-K tail of the QKV projection of short prompts (N = 3072): thread
+// The split-K tail of the QKV projection of short calls (N = 3072): thread
 // (t, j) takes RoPE pairs 2j and 2j + 1 of token row t, i.e. columns 4j .. 4j + 3
 // (dims d, d + 32, d + 1, d + 33 of one head, d = 2j mod 32), in one 16-byte
 // load per split: each column summed over the SPLITS fp32 partials in split
-// order and rounded to bf16, RoPE on the q and k pairs as the QKV GEMM's
+// order (MIXED: as in pf_reduce_norm) and rounded to bf16, RoPE on the q and k pairs as the QKV GEMM's
 // epilogue does it, q to the q buffer and k and v to the caches at row
 // p0 + t, two bf16 per 4-byte store. Grid (T, QKV_PAIRS / 2 / NT).
-template <int SPLITS>
+template <int SPLITS, bool MIXED>
 __global__ void __launch_bounds__(NT) pf_qkv_finish(const float* part, const uint16_t* rope, uint16_t* q,
                                                     uint16_t* kc, uint16_t* vc, int T, int p0, int s_max) {
   const int t = blockIdx.x, j = blockIdx.y * NT + (int)threadIdx.x;
@@ -383,16 +419,16 @@ __global__ void __launch_bounds__(NT) pf_qkv_finish(const float* part, const uin
 #pragma unroll
   for (int sp = 0; sp < SPLITS; ++sp)
     pv[sp] = *reinterpret_cast<const float4*>(part + ((size_t)sp * T + t) * QKV_ROWS + 4 * j);
-  float v0 = 0.f, v1 = 0.f, v2 = 0.f, v3 = 0.f;
+  float4 v = {0.f, 0.f, 0.f, 0.f};
+  if (MIXED && pos >= EARLY_ROWS) {
 #pragma unroll
-  for (int sp = 0; sp < SPLITS; ++sp) {
-    v0 += pv[sp].x;
-    v1 += pv[sp].y;
-    v2 += pv[sp].z;
-    v3 += pv[sp].w;
+    for (int sp = 0; sp + 1 < SPLITS; sp += 2) v = sum4(v, sum4(pv[sp], pv[sp + 1]));
+  } else {
+#pragma unroll
+    for (int sp = 0; sp < SPLITS; ++sp) v = sum4(v, pv[sp]);
   }
   // pair 2j: (x[d], x[d + 32]) = (a0, b0); pair 2j + 1: (x[d + 1], x[d + 33]) = (a1, b1)
-  const float a0 = rbf(v0), b0 = rbf(v1), a1 = rbf(v2), b1 = rbf(v3);
+  const float a0 = rbf(v.x), b0 = rbf(v.y), a1 = rbf(v.z), b1 = rbf(v.w);
   float o00 = a0, o01 = b0, o10 = a1, o11 = b1;
   if (pr < Q_PAIRS + K_PAIRS) {
     const uint16_t* rrow = rope + (size_t)pos * (2 * HD);
@@ -445,11 +481,13 @@ struct AttnArgs {
   uint16_t* att;         // A-tile order [T16][2048]
   float* part;           // key splits: o of (split, token, q head) [64], then (max, sum) of each
   int T, p0, s_max;
-  int split;             // keys per split (a multiple of KB)
+  int b0, nb;            // the launch's blocks of tokens
+  int split;             // keys per split (a multiple of KB); short calls: short_split instead
   int nsplit;
 };
+// The rows a launch of pf_attn is for: any, or a short call's (early: before EARLY_ROWS).
+enum : int { ANY = 0, SHORT_EARLY = 1, SHORT_LATE = 2 };
 
-constexpr int EARLY = 128;            // prompts within so many rows: fixed order of all sums (attn_run)
 constexpr int KB = 64;                // keys per step
 constexpr int VT_LD = KB + 8;         // bf16 per row (one dim) of the transposed V tile: 144 bytes
 constexpr int ANS = 3;                // steps of K and V in LDS
@@ -463,6 +501,16 @@ struct AttnTile {
   u32x4 k[8][64];
   uint16_t vt[HD][VT_LD];
 };
+
+// Short calls: keys per split for the token at `row` of the cache, the same for the
+// 16 rows of an aligned block: all of them up to SHORT_WHOLE, else an eighth in
+// steps of KB (it grows every 512 rows, between blocks).
+constexpr int SHORT_WHOLE = 640;
+__host__ __device__ inline int short_split(int row) {
+  const int n = (row | 15) + 1;   // keys the block's last token sees
+  return n <= SHORT_WHOLE ? SHORT_WHOLE : max(4 * KB, (n + 8 * KB - 1) / (8 * KB) * KB);
+}
+static_assert((size_t)8 * SHORT_TOKENS * NQ * (HD + 2) * 4 <= PART_BYTES, "eight parts of each token fit");
 
 // Causal attention. Token t of the sequence (position p0 + t) attends to cache
 // rows [0, p0 + t], its own row included (written by the QKV projection before
@@ -483,19 +531,22 @@ struct AttnTile {
 // transposed by 2-byte stores: 3001 tokens 112 -> 69 us, 1100 tokens 28.8 -> 23.
 // Three and four tiles per wave are slower than two (84 and 94 us at 3001).
 //
-// HALVES: the running maximum moves every 32 keys, and scores are exponentiated
-// as they are: the outputs of 32-key steps bit for bit (attn_run).
-template <int NTL, bool SPLIT, bool HALVES>
+// Short calls: a workgroup's tokens are those of 16 rows of the cache from a
+// multiple of 16 on, and their key split is those rows' (short_split). For the rows
+// before EARLY_ROWS the running maximum moves every 32 keys, scores exponentiated
+// as they are.
+template <int NTL, bool SPLIT, int ROWS>
 __global__ void __launch_bounds__(NT, NTL > 2 ? 2 : 3) pf_attn(AttnArgs a) {
   __shared__ AttnTile L[ANS];
   const int h = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), tid_ = threadIdx.x, lane = tid_ & 63;
-  const int nblk = (a.T + 16 * NTL - 1) / (16 * NTL);
+  const int skew = ROWS == ANY ? 0 : a.p0 & 15;   // rows of the call's first block before its first token
   const int g = blockIdx.x & 7;                // kv head
   static_assert(NKV == 8, "a kv head per XCD");
-  const int tb = nblk - 1 - ((int)blockIdx.x >> 3) % nblk, sp = ((int)blockIdx.x >> 3) / nblk;
-  const int t0 = tb * 16 * NTL;
+  const int tb = a.b0 + a.nb - 1 - ((int)blockIdx.x >> 3) % a.nb, sp = ((int)blockIdx.x >> 3) / a.nb;
+  const int t0 = tb * 16 * NTL - skew;
   const int k_end = a.p0 + min(t0 + 16 * NTL, a.T);
-  const int key0 = SPLIT ? sp * a.split : 0, n_keys = SPLIT ? min(k_end, key0 + a.split) : k_end;
+  const int split = ROWS == ANY ? a.split : short_split(a.p0 + t0);
+  const int key0 = SPLIT ? sp * split : 0, n_keys = SPLIT ? min(k_end, key0 + split) : k_end;
   if (SPLIT && key0 >= k_end) return;          // (the merge knows)
   const int col = lane & 15, q4 = lane >> 4, hq = GQA * g + h;
   const rsrc_t rq = make_rsrc(a.q, (size_t)a.T * H * 2);
@@ -505,7 +556,7 @@ __global__ void __launch_bounds__(NT, NTL > 2 ? 2 : 3) pf_attn(AttnArgs a) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const int tq = t0 + 16 * j + col;
-      qv[j][s] = ld16(rq, tq < a.T ? (uint32_t)(((size_t)tq * H + hq * HD + 32 * s + q4 * 8) * 2) : OOB);
+      qv[j][s] = ld16(rq, (uint32_t)tq < (uint32_t)a.T ? (uint32_t)(((size_t)tq * H + hq * HD + 32 * s + q4 * 8) * 2) : OOB);
     }
   const rsrc_t rk = make_rsrc(a.kc + (size_t)g * a.s_max * HD, (size_t)a.s_max * HD * 2);
   const rsrc_t rv = make_rsrc(a.vc + (size_t)g * a.s_max * HD, (size_t)a.s_max * HD * 2);
@@ -586,8 +637,8 @@ __global__ void __launch_bounds__(NT, NTL > 2 ? 2 : 3) pf_attn(AttnArgs a) {
     }
   };
   auto compute = [&](int k0, const AttnTile& cur) {
-    if constexpr (HALVES) {
-      static_assert(NTL == 1 && !SPLIT, "one tile, all keys");
+    if constexpr (ROWS == SHORT_EARLY) {
+      static_assert(NTL == 1 && !SPLIT && EARLY_ROWS <= SHORT_WHOLE, "one tile, all keys");
       compute_half(k0, 0, cur);
       compute_half(k0, 1, cur);
       return;
@@ -680,7 +731,7 @@ __global__ void __launch_bounds__(NT, NTL > 2 ? 2 : 3) pf_attn(AttnArgs a) {
   for (int j = 0; j < NTL; ++j) {
     const int tq = t0 + 16 * j + col;
     const float l_tot = add_xor32(add_xor16(l_run[j]));
-    if (tq >= a.T) continue;
+    if ((uint32_t)tq >= (uint32_t)a.T) continue;
     if constexpr (SPLIT) {
       const size_t at = ((size_t)sp * a.T + tq) * NQ + hq, n = (size_t)a.nsplit * a.T * NQ;
 #pragma unroll
@@ -700,13 +751,16 @@ __global__ void __launch_bounds__(NT, NTL > 2 ? 2 : 3) pf_attn(AttnArgs a) {
 }
 
 // The attention output from the splits' parts: 16 lanes per (token, q head),
-// four dims each; the splits that hold keys of the token's workgroup, in order.
-__global__ void __launch_bounds__(NT) pf_attn_merge(AttnArgs a, int tokens_per_wg) {
+// four dims each; the splits that hold keys of the token's workgroup (SHORT: of
+// the token), in order.
+template <bool SHORT>
+__global__ void __launch_bounds__(NT) pf_attn_merge(AttnArgs a) {
   const int i = (int)blockIdx.x * (NT / 16) + ((int)threadIdx.x >> 4), t = i / NQ, hq = i % NQ;
   const int d = ((int)threadIdx.x & 15) * 4;
   if (t >= a.T) return;
-  const int k_end = a.p0 + min((t / tokens_per_wg + 1) * tokens_per_wg, a.T);
-  const int ns = min((k_end + a.split - 1) / a.split, a.nsplit);
+  const int k_end = SHORT ? a.p0 + t + 1 : a.p0 + min((t / 16 + 1) * 16, a.T);
+  const int split = SHORT ? short_split(a.p0 + t) : a.split;
+  const int ns = min((k_end + split - 1) / split, a.nsplit);
   const float2* ml = reinterpret_cast<const float2*>(a.part + (size_t)a.nsplit * a.T * NQ * HD);
   float M = -INFINITY;
   for (int s = 0; s < ns; ++s) M = fmaxf(M, ml[((size_t)s * a.T + t) * NQ + hq].x);
@@ -724,11 +778,12 @@ __global__ void __launch_bounds__(NT) pf_attn_merge(AttnArgs a, int tokens_per_w
       uint2{pack_bf2(o[0] * inv, o[1] * inv), pack_bf2(o[2] * inv, o[3] * inv)};
 }
 
-template <int NTL, bool SPLIT, bool HALVES = false>
+template <int NTL, bool SPLIT, int ROWS = ANY>
 void attn_launch(const AttnArgs& a, hipStream_t st) {
-  const int nblk = (a.T + 16 * NTL - 1) / (16 * NTL);
-  hipLaunchKernelGGL((pf_attn<NTL, SPLIT, HALVES>), dim3(nblk * NKV * (SPLIT ? a.nsplit : 1)), dim3(NT), 0, st, a);
-  if (SPLIT) hipLaunchKernelGGL(pf_attn_merge, dim3((a.T * NQ + NT / 16 - 1) / (NT / 16)), dim3(NT), 0, st, a, 16 * NTL);
+  static_assert(NTL == 1 || (!SPLIT && ROWS == ANY), "pf_attn_merge and short calls count 16 tokens per workgroup");
+  hipLaunchKernelGGL((pf_attn<NTL, SPLIT, ROWS>), dim3(a.nb * NKV * (SPLIT ? a.nsplit : 1)), dim3(NT), 0, st, a);
+  if (SPLIT)
+    hipLaunchKernelGGL(pf_attn_merge<ROWS != ANY>, dim3((a.T * NQ + NT / 16 - 1) / (NT / 16)), dim3(NT), 0, st, a);
 }
 // Tiles of 16 tokens up to 2048 tokens, of 32 above (one 16-token tile per wave
 // against two: 2048 tokens 44 against 47 us, 3001 tokens 92 against 71). Few
@@ -738,14 +793,29 @@ void attn_launch(const AttnArgs& a, hipStream_t st) {
 // (33 tokens at 4000 rows: 55 us whole, 17.5 in 8 parts; at 700 rows 13.6 and
 // 11.0). Splits begin at multiples of 64 keys of the cache.
 //
-// Prompts within the first EARLY rows take the running maximum over 32 keys
-// (HALVES) and fixed K splits (gemm_plan): the bits of the 32-key kernel and its
-// splits, whatever a call's number of tokens. One layer (before: that kernel, its GEMMs):
-// 20 tokens 73.6 -> 45.8 us, 64 83.7 -> 53.6; 128 tokens take 72 us, about 65 with
-// the splits of later rows (16.8 MB of partials instead of 8.4).
+// Short calls split a token's keys by its row alone (short_split); a call across
+// EARLY_ROWS takes a launch for the rows on either side (no keys are split there).
 void attn_run(AttnArgs a, hipStream_t st) {
-  if (a.p0 + a.T <= EARLY) return attn_launch<1, false, true>(a, st);
-  const int n_keys = a.p0 + a.T, wgs = (a.T + 15) / 16 * NKV;
+  a.b0 = 0;
+  if (a.T <= SHORT_TOKENS) {
+    const int base = a.p0 & ~15, nb = (a.p0 + a.T - base + 15) / 16;
+    const int early = min(max((EARLY_ROWS - base) / 16, 0), nb);
+    a.nsplit = 1;
+    for (int row = base; row < a.p0 + a.T; row += 16)
+      a.nsplit = max(a.nsplit, (min(row + 16, a.p0 + a.T) + short_split(row) - 1) / short_split(row));
+    if (early) {
+      a.nb = early;
+      attn_launch<1, false, SHORT_EARLY>(a, st);
+    }
+    a.b0 = early;
+    a.nb = nb - early;
+    if (!a.nb) return;
+    if (a.nsplit == 1) return attn_launch<1, false, SHORT_LATE>(a, st);
+    return attn_launch<1, true, SHORT_LATE>(a, st);
+  }
+  static_assert(EARLY_ROWS % 16 == 0 && EARLY_ROWS + SHORT_TOKENS <= SHORT_WHOLE, "early and split rows in no one call");
+  a.nb = (a.T + 15) / 16;
+  const int n_keys = a.p0 + a.T, wgs = a.nb * NKV;
   const int most = (int)(PART_BYTES / ((size_t)NQ * (HD + 2) * 4)) / a.T;   // splits whose parts fit
   const int ns = min(min(8, 3 * 256 / wgs), most);
   if (ns >= 2) {
@@ -757,8 +827,9 @@ void attn_run(AttnArgs a, hipStream_t st) {
       return attn_launch<1, true>(a, st);
     }
   }
-  if (a.T <= 2048) attn_launch<1, false>(a, st);
-  else attn_launch<2, false>(a, st);
+  if (a.T <= 2048) return attn_launch<1, false>(a, st);
+  a.nb = (a.T + 31) / 32;
+  attn_launch<2, false>(a, st);
 }
 
 size_t ws_per_token() { return (size_t)H * 2 * 5 + (size_t)INTER * 2; }
@@ -777,85 +848,88 @@ constexpr GemmTile TILES[] = {{64, 64, 2.73f, 0.50f, 0.13f},    {128, 128, 0.34f
                               {192, 128, -1.88f, 8.42f, 0.32f}, {256, 128, -0.94f, 10.66f, 0.37f},
                               {192, 128, 8.99f, -0.77f, 0.33f}, {160, 256, 0.30f, 10.96f, 0.45f},
                               {256, 256, -2.26f, 19.51f, 0.54f}};
-// (built with every epilogue up to here: the others hardly ever win for N = 2048, or with K split)
-constexpr int TILES_RES = 4, TILES_PART = 3, TILES_ALL = sizeof(TILES) / sizeof(TILES[0]);
+// The tiles each epilogue is built on: [first, end) of TILES. Those above 256x128
+// hardly ever win for N = 2048, those above 192x128 with K split; short calls are
+// the fastest on 64x64 in pairs.
+struct TileRange {
+  int first, end;
+};
+constexpr TileRange tiles_of(int epi) {
+  return epi == EPI_RES ? TileRange{0, 4} : epi == EPI_PART ? TileRange{0, 3} : epi == EPI_PAIR ? TileRange{0, 1}
+                                                                                               : TileRange{0, 7};
+}
 
-template <int EPI, int MI, int NI, int WM, int WN, int NS>
-void gemm_launch(const GemmArgs& g, const GemmTile& t, hipStream_t st) {
-  hipLaunchKernelGGL((pf_gemm<EPI, MI, NI, WM, WN, NS>), dim3(g.mt * (g.N / t.tn) * g.splits), dim3(64 * WM * WN), 0, st,
-                     g);
+template <int EPI, int TILE, int MI, int NI, int WM, int WN, int NS>
+void gemm_launch(const GemmArgs& g, hipStream_t st) {
+  constexpr GemmTile t = TILES[TILE];
+  static_assert(t.tm == 16 * MI * WM && t.tn == 16 * NI * WN, "the tile of TILES");
+  if constexpr (TILE >= tiles_of(EPI).first && TILE < tiles_of(EPI).end)
+    hipLaunchKernelGGL((pf_gemm<EPI, MI, NI, WM, WN, NS>), dim3(g.mt * (g.N / t.tn) * g.splits), dim3(64 * WM * WN), 0,
+                       st, g);
 }
 template <int EPI>
 void gemm_run(GemmArgs g, int tile, hipStream_t st) {
-  const GemmTile& t = TILES[tile];
-  g.mt = (g.M + t.tm - 1) / t.tm;
+  g.mt = (g.M + TILES[tile].tm - 1) / TILES[tile].tm;
   switch (tile) {
-    case 0: return gemm_launch<EPI, 2, 2, 2, 2, 6>(g, t, st);
-    case 1: return gemm_launch<EPI, 2, 4, 4, 2, 6>(g, t, st);
-    case 2: return gemm_launch<EPI, 3, 4, 4, 2, 5>(g, t, st);
-  }
-  if constexpr (EPI != EPI_PART) {
-    if (tile == 3) return gemm_launch<EPI, 4, 4, 4, 2, 4>(g, t, st);
-    if constexpr (EPI != EPI_RES) {
-      if (tile == 4) return gemm_launch<EPI, 6, 4, 2, 2, 4>(g, t, st);
-      if (tile == 5) return gemm_launch<EPI, 5, 4, 2, 4, 4>(g, t, st);
-      if (tile == 6) return gemm_launch<EPI, 8, 4, 2, 4, 4>(g, t, st);
-    }
+    case 0: return gemm_launch<EPI, 0, 2, 2, 2, 2, 6>(g, st);
+    case 1: return gemm_launch<EPI, 1, 2, 4, 4, 2, 6>(g, st);
+    case 2: return gemm_launch<EPI, 2, 3, 4, 4, 2, 5>(g, st);
+    case 3: return gemm_launch<EPI, 3, 4, 4, 4, 2, 4>(g, st);
+    case 4: return gemm_launch<EPI, 4, 6, 4, 2, 2, 4>(g, st);
+    case 5: return gemm_launch<EPI, 5, 5, 4, 2, 4, 4>(g, st);
+    case 6: return gemm_launch<EPI, 6, 8, 4, 2, 4, 4>(g, st);
   }
 }
 
-// Tile and K splits of a projection of M tokens: the least estimated time, a
-// split's partials and tail included (tail: us of a tail kernel that only a
-// split needs; the partials are written and read once at 3-4 TB/s). An output
-// is the same whatever the tile (its k-steps are summed in order) but not
-// whatever the split, so the splits are those of M rounded up to 128 tokens
-// (of 64 for the first 128, where short turns lie): a prompt of up to 128
-// tokens gives the same bits in any chunks. Prompts within the first EARLY rows
-// have fixed splits (attn_run), EARLY_QKV and EARLY_RES.
-constexpr int EARLY_QKV = 8, EARLY_RES = 16;
-struct GemmPlan {
-  int tile, splits;
-};
-// The splits the tails are built for; f(std::integral_constant<int, splits>).
-// (3 and 5 fill the device where 2 and 4 leave a quarter of it idle and the
-// partials of 8 do not fit: the down projection of 383 tokens on 240 workgroups
-// instead of 192 takes 20.4 us instead of 23.1, its tail 6.0 instead of 5.8; the
-// parts of K then differ by one pair of k-steps.)
-constexpr int SPLITS[] = {2, 3, 4, 5, 8, 16};
-template <class F>
-void with_splits(int splits, F&& f) {
-  switch (splits) {
-    case 2: return f(std::integral_constant<int, 2>{});
-    case 3: return f(std::integral_constant<int, 3>{});
-    case 4: return f(std::integral_constant<int, 4>{});
-    case 5: return f(std::integral_constant<int, 5>{});
-    case 8: return f(std::integral_constant<int, 8>{});
-    case 16: return f(std::integral_constant<int, 16>{});
-  }
-}
-float gemm_us(const GemmTile& t, int M, int N, int K, int splits, float tail) {
+// The estimated time of a projection of M tokens. A split adds what it moves (its
+// partials' bytes at 7 TB/s: a weight that chooses well, not a bandwidth, since the
+// fitted times hold the GEMM's own stores) less 0.5 us, as its tail takes the place
+// of pf_norm.
+float gemm_us(const GemmTile& t, int M, int N, int K, int splits) {
   const int wg = (M + t.tm - 1) / t.tm * (N / t.tn) * splits;
   const float rounds = t.tm == 64 ? fmaxf(1.f, (float)wg / 256.f) : (float)((wg + 255) / 256);
   const float us = t.fixed + rounds * (t.round + t.kstep * (float)((K / 64 + splits - 1) / splits * 2));
-  return splits == 1 ? us : us + tail + (float)splits * (float)M * (float)N * 4.f / 7e6f;
+  return splits == 1 ? us : us - 0.5f + (float)splits * (float)M * (float)N * 4.f / 7e6f;
 }
-GemmPlan gemm_plan(int M, int N, int K, int tiles, size_t part_bytes, float tail, int fixed = 0) {
-  GemmPlan best = {0, fixed ? fixed : 1};
-  const int most = (M + 127) / 128 * 128, Ms = most <= 128 ? 64 : most;
-  for (int sp : SPLITS) {
-    if (fixed || (size_t)sp * most * N * 4 > part_bytes) break;
-    auto least = [&](int s) {
-      const int n = s > 1 ? TILES_PART : tiles;
-      float us = gemm_us(TILES[0], Ms, N, K, s, tail);
-      for (int i = 1; i < n; ++i) us = fminf(us, gemm_us(TILES[i], Ms, N, K, s, tail));
-      return us;
-    };
-    if (least(sp) < least(best.splits)) best.splits = sp;
-  }
-  const int n = best.splits > 1 ? TILES_PART : tiles;
-  for (int i = 1; i < n; ++i)
-    if (gemm_us(TILES[i], M, N, K, best.splits, tail) < gemm_us(TILES[best.tile], M, N, K, best.splits, tail)) best.tile = i;
+// The tile for it among an epilogue's: the least estimated time.
+int gemm_tile(int epi, int M, int N, int K, int splits) {
+  const TileRange r = tiles_of(epi);
+  int best = r.first;
+  for (int i = r.first + 1; i < r.end; ++i)
+    if (gemm_us(TILES[i], M, N, K, splits) < gemm_us(TILES[best], M, N, K, splits)) best = i;
   return best;
+}
+// The K splits of an N = 2048 projection of M > SHORT_TOKENS tokens whose partials
+// fit in part_bytes: the least estimated time. An output is the same whatever the
+// tile (its k-steps are summed in order) but not whatever the split, so it is that of
+// M rounded up to 128 tokens. (3 and 5 fill the device where 2 and 4 leave a
+// quarter of it idle and the partials of 8 do not fit: the down projection of 383
+// tokens on 240 workgroups instead of 192 takes 20.4 us instead of 23.1, its tail
+// 6.0 instead of 5.8; the parts of K then differ by one pair of k-steps.)
+int gemm_splits(int M, int N, int K, size_t part_bytes) {
+  const int most = (M + 127) / 128 * 128;
+  auto least = [&](int s) {
+    const int epi = s == 1 ? EPI_RES : EPI_PART;
+    return gemm_us(TILES[gemm_tile(epi, most, N, K, s)], most, N, K, s);
+  };
+  int best = 1;
+  for (int sp : {2, 3, 4, 5, 8})
+    if ((size_t)sp * most * N * 4 <= part_bytes && least(sp) < least(best)) best = sp;
+  return best;
+}
+// Short calls cut K into SHORT_QKV or SHORT_RES parts. From row EARLY_ROWS on a
+// workgroup takes two of them, each summed from zero, and stores the sum (EPI_PAIR:
+// half the partials); an earlier call stores each part, and where it reaches past
+// EARLY_ROWS its tails add the pairs there (MIXED). A row's sums are the same.
+// One layer, 33 tokens at row 700: 51 us as with the splits of least estimated
+// time (5, 8 and 8), 128 tokens at row 200: 61 us; every part stored and every
+// maximum over 32 keys there: 55 and 71 us.
+constexpr int SHORT_QKV = 8, SHORT_RES = 16;
+void gemm_short(GemmArgs g, int parts, hipStream_t st) {
+  const bool pairs = g.p0 >= EARLY_ROWS;
+  g.splits = pairs ? parts / 2 : parts;
+  if (pairs) gemm_run<EPI_PAIR>(g, 0, st);
+  else gemm_run<EPI_PART>(g, gemm_tile(EPI_PART, g.M, g.N, g.K, parts), st);
 }
 
 }  // namespace
@@ -890,29 +964,48 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
   uint16_t* q = att + c16 * H;
   float* part = reinterpret_cast<float*>(q + c16 * H);
   const int L = a->n_layers, l0 = a->first_layer;
+  // A short call's parts of K: f(number of partials, whether the tail adds pairs).
+  auto with_parts = [](auto parts, const GemmArgs& g, auto&& f) {
+    if (g.p0 >= EARLY_ROWS) return f(std::integral_constant<int, parts.value / 2>{}, std::false_type{});
+    if (g.p0 + g.M <= EARLY_ROWS) return f(parts, std::false_type{});
+    return f(parts, std::true_type{});
+  };
+  // The split-K tail of an N = 2048 projection: SPLITS partials, summed as pf_reduce_norm says.
+  auto reduce = [&](auto splits, auto mixed, const GemmArgs& g, const uint16_t* res, uint16_t* out, bool norm) {
+    hipLaunchKernelGGL((pf_reduce_norm<splits.value, mixed.value>), dim3(g.M), dim3(NT), 0, st, (const float*)g.part, res,
+                       out, norm ? xn : (uint16_t*)nullptr, g.M, g.p0);
+  };
   // An N = 2048 projection (O: K = 2048, down: K = 8192) of T tokens with the
   // residual add, followed by the RMSNorm of its output into xn if `norm`:
   // as one GEMM with the add in its epilogue plus pf_norm, or, where few tiles
   // would leave the device idle, split over K into fp32 partials that
   // pf_reduce_norm sums (in split order), adds and normalises.
-  auto res_gemm = [&](GemmArgs g, const uint16_t* res, uint16_t* out, bool norm, int T, float* parts, size_t part_bytes,
-                      bool early) {
-    const GemmPlan pl = gemm_plan(T, g.N, g.K, TILES_RES, part_bytes, -0.5f, early ? EARLY_RES : 0);
-    g.splits = pl.splits;
-    if (pl.splits == 1) {
+  auto res_gemm = [&](GemmArgs g, const uint16_t* res, uint16_t* out, bool norm, float* parts, size_t part_bytes) {
+    const auto plain = std::false_type{};
+    g.part = parts;
+    if (g.M <= SHORT_TOKENS) {
+      gemm_short(g, SHORT_RES, st);
+      return with_parts(std::integral_constant<int, SHORT_RES>{}, g,
+                        [&](auto n, auto mixed) { reduce(n, mixed, g, res, out, norm); });
+    }
+    g.splits = gemm_splits(g.M, g.N, g.K, part_bytes);
+    const int tile = gemm_tile(g.splits == 1 ? EPI_RES : EPI_PART, g.M, g.N, g.K, g.splits);
+    if (g.splits == 1) {
       g.res = res;
       g.out = out;
-      gemm_run<EPI_RES>(g, pl.tile, st);
+      gemm_run<EPI_RES>(g, tile, st);
       if (norm)
-        hipLaunchKernelGGL(pf_norm, dim3((unsigned)((T + NWAVE - 1) / NWAVE)), dim3(NT), 0, st, (const uint16_t*)out,
-                           (const int32_t*)nullptr, (const uint16_t*)nullptr, (uint16_t*)nullptr, xn, T);
-    } else {
-      g.part = parts;
-      gemm_run<EPI_PART>(g, pl.tile, st);
-      uint16_t* xn_out = norm ? xn : nullptr;
-      with_splits(pl.splits, [&](auto n) {
-        hipLaunchKernelGGL(pf_reduce_norm<n.value>, dim3(T), dim3(NT), 0, st, (const float*)parts, res, out, xn_out, T);
-      });
+        hipLaunchKernelGGL(pf_norm, dim3((unsigned)((g.M + NWAVE - 1) / NWAVE)), dim3(NT), 0, st, (const uint16_t*)out,
+                           (const int32_t*)nullptr, (const uint16_t*)nullptr, (uint16_t*)nullptr, xn, g.M);
+      return;
+    }
+    gemm_run<EPI_PART>(g, tile, st);
+    switch (g.splits) {
+      case 2: return reduce(std::integral_constant<int, 2>{}, plain, g, res, out, norm);
+      case 3: return reduce(std::integral_constant<int, 3>{}, plain, g, res, out, norm);
+      case 4: return reduce(std::integral_constant<int, 4>{}, plain, g, res, out, norm);
+      case 5: return reduce(std::integral_constant<int, 5>{}, plain, g, res, out, norm);
+      case 8: return reduce(std::integral_constant<int, 8>{}, plain, g, res, out, norm);
     }
   };
   // Every chunk starts again from the embeddings of its own tokens; the rows
@@ -920,7 +1013,6 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
   // only its QKV GEMM unless the hidden state is asked for.
   for (int c0 = 0; c0 < a->n_tokens; c0 += cap) {
     const int T = min(cap, a->n_tokens - c0), p0 = a->start_pos + c0;
-    const bool early = p0 + T <= EARLY;
     hipLaunchKernelGGL(pf_norm, dim3((T + NWAVE - 1) / NWAVE), dim3(NT), 0, st, (const uint16_t*)nullptr,
                        a->tokens + c0, static_cast<const uint16_t*>(w->embed), x, xn, T);
     for (int li = 0; li < L; ++li) {
@@ -944,20 +1036,16 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
       g.out = q;
       g.kc = kc;
       g.vc = vc;
-      const GemmPlan qp = gemm_plan(T, QKV_ROWS, H, TILES_ALL, PART_BYTES, 4.5f, early ? EARLY_QKV : 0);
-      g.splits = qp.splits;
-      if (qp.splits == 1) {
-        gemm_run<EPI_QKV>(g, qp.tile, st);
-      } else {   // short prompts: split over K, RoPE and the scatter in the tail
+      if (T > SHORT_TOKENS) {
+        gemm_run<EPI_QKV>(g, gemm_tile(EPI_QKV, T, QKV_ROWS, H, 1), st);
+      } else {   // split over K, RoPE and the scatter in the tail
         g.part = part;
-        gemm_run<EPI_PART>(g, qp.tile, st);
+        gemm_short(g, SHORT_QKV, st);
         const uint16_t* rope = static_cast<const uint16_t*>(w->rope);
-        const dim3 fg(T, QKV_PAIRS / 2 / NT);
-        with_splits(qp.splits, [&](auto n) {
-          hipLaunchKernelGGL(pf_qkv_finish<n.value>, fg, dim3(NT), 0, st, (const float*)part, rope, q, kc, vc, T, p0,
-                             a->s_max);
+        with_parts(std::integral_constant<int, SHORT_QKV>{}, g, [&](auto n, auto mixed) {
+          hipLaunchKernelGGL((pf_qkv_finish<n.value, mixed.value>), dim3(T, QKV_PAIRS / 2 / NT), dim3(NT), 0, st,
+                             (const float*)part, rope, q, kc, vc, T, p0, a->s_max);
         });
-        g.splits = 1;
       }
       if (tail) break;   // the last layer's K/V rows are all the caller needs
       AttnArgs aa;
@@ -976,15 +1064,14 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
       g.N = H;
       g.K = H;
       g.kc = g.vc = nullptr;
-      res_gemm(g, x, h1, true, T, part, PART_BYTES, early);
+      res_gemm(g, x, h1, true, part, PART_BYTES);
       // gate/up + SwiGLU -> act
       g.a = xn;
       g.b = Wgu + (size_t)l * 2 * INTER * H;
       g.N = 2 * INTER;
       g.K = H;
       g.out = act;
-      g.splits = 1;
-      gemm_run<EPI_SWIGLU>(g, gemm_plan(T, g.N, g.K, TILES_ALL, 0, 0.f).tile, st);
+      gemm_run<EPI_SWIGLU>(g, gemm_tile(EPI_SWIGLU, T, g.N, g.K, 1), st);
       // down projection + residual -> x (the next layer's input) and its RMSNorm -> xn,
       // or the caller's hidden state after the last layer
       g.a = act;
@@ -994,8 +1081,8 @@ hipError_t prefill_launch(const mk_weights* w, const mk_prefill_args* a, int cap
       // (att and q hold nothing any more and lie before `part`)
       float* down_part = reinterpret_cast<float*>(att);
       const size_t down_bytes = PART_BYTES + (size_t)T * H * 2 * 2;
-      if (li + 1 < L) res_gemm(g, h1, x, true, T, down_part, down_bytes, early);
-      else res_gemm(g, h1, static_cast<uint16_t*>(a->hidden_out) + (size_t)c0 * H, false, T, down_part, down_bytes, early);
+      if (li + 1 < L) res_gemm(g, h1, x, true, down_part, down_bytes);
+      else res_gemm(g, h1, static_cast<uint16_t*>(a->hidden_out) + (size_t)c0 * H, false, down_part, down_bytes);
     }
   }
   return hipGetLastError();

@@ -116,8 +116,7 @@ def test_layer_at_row_count(layer, n, start):
 @pytest.mark.parametrize("cut", [1, 32, 63, 64])
 def test_prompt_within_128_rows_in_any_chunks(layer, n, cut):
     """Whole or cut in two, a prompt within the first 128 rows gives the same
-    bits: its K splits and the attention's 32-key steps do not depend on how
-    many tokens a call has."""
+    bits."""
     import mk_lib
     if cut >= n:
         pytest.skip("nothing to cut")
@@ -130,3 +129,25 @@ def test_prompt_within_128_rows_in_any_chunks(layer, n, cut):
     torch.cuda.synchronize()
     assert torch.equal(out.view(torch.int16), out2.view(torch.int16))
     assert torch.equal(kv.view(torch.int16), kv2.view(torch.int16))
+
+
+@pytest.mark.parametrize("start", [1, 100, 250, 620, 700, 1999, 3000, 4070])
+def test_short_turn_in_any_pieces(layer, start):
+    """A turn of up to 128 tokens, cut into any smaller calls, gives the same bits
+    at any row: the order of all of a token's sums follows from its row alone. The
+    starts put the turn across row 128, where that order changes, across rows where
+    the split of the keys changes (640, 2048, 3072, 4096) and across none, on and off
+    the 16-row blocks."""
+    import mk_lib
+    n = 128
+    out, kv = run(layer, n, start, layer["tiled"])
+    ws = mk_lib.prefill_workspace(n, "cuda")
+    for cuts in ((64,), (1, 2, 19, 33, 90), tuple(range(7, n, 7))):
+        kv2 = layer["kv"].clone()
+        out2 = torch.empty_like(out)
+        for a, b in zip((0,) + cuts, cuts + (n,)):
+            mk_lib.prefill(layer["tiled"], layer["ids"][a:b].clone(), [kv2[0]], [kv2[1]], start + a, ws,
+                           hidden_out=out2[a:b])
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), out2.view(torch.int16)), cuts
+        assert torch.equal(kv.view(torch.int16), kv2.view(torch.int16)), cuts
