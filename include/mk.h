@@ -226,7 +226,7 @@ int mk_sample(const mk_sample_args *a);
  * rows' first pass then runs on many workgroups instead of one per row. Same
  * results. Calls that overlap in time need scratch of their own. scratch NULL:
  * mk_sample. MK_ERR_WORKSPACE if it is too small. mk_sample_scratch_bytes is 0
- * where no scratch is used (vocab up to 4096, or above 2097152).
+ * where no scratch is used (vocab up to 32768, or above 2097152).
  */
 size_t mk_sample_scratch_bytes(int32_t batch, int32_t vocab);
 int mk_sample_with_scratch(const mk_sample_args *a, void *scratch, size_t scratch_bytes);

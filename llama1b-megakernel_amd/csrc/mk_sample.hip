@@ -29,8 +29,9 @@
 // tokens are looked at again:
 //   1. mk_group_max_kernel (with scratch): the row as at most 8192 groups of
 //      4 * 2^s consecutive logits (16 for 128256); the largest key of each
-//      group to scratch. Without scratch the row's one workgroup does this
-//      itself, into LDS;
+//      group to scratch. Without scratch, and in rows of up to SOLO logits, the
+//      row's one workgroup does this itself, into LDS (a greedy row's just takes
+//      the argmax);
 //   2. mk_sample_kernel, one 1024-thread workgroup per row: a key L that at
 //      least k group maxima reach, from a histogram of the maxima over 2048
 //      equal key ranges (bisection within one range where that is too coarse).
@@ -108,6 +109,12 @@ constexpr int BINS = 2048;               // key ranges of a histogram
 constexpr int CROWD = 32;                // candidates in one key range that are still ordered by counting
 constexpr int NG = 8;                    // group maxima per thread
 constexpr int MAX_GROUPS = NG * ST;
+// Longest row that its own workgroup reads alone, with scratch too. The first
+// kernel costs 2 us and its launch; one workgroup's pass over 32768 logits is about
+// as long. With scratch against without, batch 1: 8192 logits greedy 6.3, 3.4 us,
+// top-k 50 11.9, 10.7; 32768 greedy 6.4, 6.0, top-k 50 13.4, 13.7; 48000 6.7, 7.6
+// and 13.9, 16.6 (and a call without it takes 4 us less of the host's time).
+constexpr int SOLO = 32768;
 constexpr int GT = 256;                  // threads of the group maximum kernel
 constexpr int GSEG = 4;                  // 256-logit segments per wave of it
 
@@ -501,14 +508,17 @@ __global__ void __launch_bounds__(ST) mk_sample_kernel(SParams p, const uint32_t
   uint32_t gm[NG];
 #pragma unroll
   for (int j = 0; j < NG; ++j) gm[j] = 0u;
-  if (gs) {
+  if (gs && (gmax || !greedy)) {
     const uint32_t* src = gmax + (size_t)row * ngroups;
     if (!gmax) {   // into the sort's LDS, not in use yet
       uint32_t* own = reinterpret_cast<uint32_t*>(L.tmp);
       static_assert(MAX_GROUPS * sizeof(uint32_t) <= sizeof(L.tmp), "group maxima in LDS");
-      const int nseg = (V + 255) / 256;
-      for (int s0 = wave; s0 < nseg; s0 += 16 * (ST / 64))
-        group_max<16>(x, V, gs, s0, ST / 64, [&](int g, uint32_t m) { own[g] = m; });
+      const int nseg = (V + 255) / 256, nw = ST / 64;
+      auto put = [&](int g, uint32_t m) { own[g] = m; };
+      if (nseg <= 4 * nw) group_max<4>(x, V, gs, wave, nw, put);
+      else if (nseg <= 8 * nw) group_max<8>(x, V, gs, wave, nw, put);
+      else
+        for (int s0 = wave; s0 < nseg; s0 += 16 * nw) group_max<16>(x, V, gs, s0, nw, put);
       __syncthreads();
 #pragma unroll
       for (int j = 0; j < NG; ++j)
@@ -527,12 +537,18 @@ __global__ void __launch_bounds__(ST) mk_sample_kernel(SParams p, const uint32_t
       const unsigned long long kv = ((unsigned long long)key << 32) | (0xffffffffu - (uint32_t)i);
       b = kv > b ? kv : b;
     };
-    if (gs) {   // the first group with the largest maximum, by its first index
+    if (gmax) {   // the first group with the largest maximum, by its first index
 #pragma unroll
       for (int j = 0; j < NG; ++j)
         if (t + j * ST < ngroups) take(gm[j], (t + j * ST) * gs);
     } else {
-      for (int i = t; i < V; i += ST) take(okey(x[i]), i);
+      const bool vec = aligned16(x);
+      for (int i = 4 * t; i < V; i += 4 * ST) {
+        uint32_t kx[4];
+        keys4(x, i, V, vec, kx);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) take(kx[e], i + e);   // (past the row: key 0, behind index 0's)
+      }
     }
     for (int o = 32; o >= 1; o >>= 1) {
       const unsigned long long v = __shfl_xor(b, o, 64);
@@ -544,7 +560,7 @@ __global__ void __launch_bounds__(ST) mk_sample_kernel(SParams p, const uint32_t
       unsigned long long m = L.best[0];
       for (int w = 1; w < ST / 64; ++w) m = L.best[w] > m ? L.best[w] : m;
       int at = (int)(0xffffffffu - (uint32_t)(m & 0xffffffffull));
-      if (gs) {   // the first logit of that group with its maximum
+      if (gmax) {   // the first logit of that group with its maximum
         const uint32_t best = (uint32_t)(m >> 32);
         for (int o = 0; o < gs; o += 64) {
           const int i = at + o + lane;
@@ -627,7 +643,7 @@ extern "C" {
 const char* mk_sample_last_error(void) { return s_msg; }
 
 size_t mk_sample_scratch_bytes(int32_t batch, int32_t vocab) {
-  const int gs = vocab > 0 ? group_size(vocab) : 0;
+  const int gs = vocab > SOLO ? group_size(vocab) : 0;
   return gs && batch > 0 ? (size_t)batch * ((vocab + gs - 1) / gs) * sizeof(uint32_t) : 0;
 }
 
@@ -658,7 +674,7 @@ int mk_sample_with_scratch(const mk_sample_args* a, void* scratch, size_t scratc
   p.stride = a->vocab_stride;
   hipStream_t st = static_cast<hipStream_t>(a->stream);
   const int gs = group_size(a->vocab);
-  uint32_t* gmax = gs ? static_cast<uint32_t*>(scratch) : nullptr;
+  uint32_t* gmax = gs && a->vocab > SOLO ? static_cast<uint32_t*>(scratch) : nullptr;
   if (gmax) {
     const int nseg = (a->vocab + 255) / 256, per = GSEG * (GT / 64);
     hipLaunchKernelGGL(mk_group_max_kernel, dim3(a->batch, (nseg + per - 1) / per), dim3(GT), 0, st, a->logits,

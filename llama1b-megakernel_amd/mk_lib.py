@@ -9,6 +9,7 @@ fallback implementation of the decode step.
 from __future__ import annotations
 
 import ctypes
+import functools
 import sys
 import weakref
 from ctypes import POINTER, c_char_p, c_int, c_int32, c_size_t, c_uint32, c_void_p
@@ -396,14 +397,19 @@ def sample(logits: torch.Tensor, params: torch.Tensor, tokens_out: torch.Tensor,
         raise ValueError("tokens_out must be int32 with at least B elements")
     a = MkSampleArgs(logits.data_ptr(), B, V, logits.stride(0), params.data_ptr(), seed & 0xFFFFFFFFFFFFFFFF,
                      _ptr(counter), tokens_out.data_ptr(), _ptr(uniforms_out), current_stream_ptr())
-    # scratch from torch's allocator: its own for every call, and ordered by the current stream
-    # (under a capture it comes from the graph's pool)
+    # scratch (long rows only) from torch's allocator: its own for every call, and ordered by the
+    # current stream (under a capture it comes from the graph's pool)
     lib = load()
-    n = lib.mk_sample_scratch_bytes(B, V)
+    n = _sample_scratch_bytes(B, V)
     scratch = torch.empty(n, dtype=torch.uint8, device=logits.device) if n else None
     rc = lib.mk_sample_with_scratch(ctypes.byref(a), _ptr(scratch), n)
     if rc != MK_OK:
-        raise MkError(rc, load().mk_sample_last_error().decode(errors="replace"))
+        raise MkError(rc, lib.mk_sample_last_error().decode(errors="replace"))
+
+
+@functools.lru_cache(maxsize=64)
+def _sample_scratch_bytes(batch: int, vocab: int) -> int:
+    return load().mk_sample_scratch_bytes(batch, vocab)
 
 
 class StepLauncher:

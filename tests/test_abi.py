@@ -198,3 +198,24 @@ def test_prefill_rejects_bad_weights(lib):
     assert lib.mk_prefill(ctypes.byref(_weights(w_gu=None)), ctypes.byref(a)) == -1
     assert lib.mk_prefill(ctypes.byref(_weights(n_layers=8)), ctypes.byref(a)) == -2
     assert lib.mk_prefill(None, ctypes.byref(a)) == -1
+
+
+@pytest.mark.parametrize("batch,vocab,groups", [
+    (1, 1, 0), (32, 4096, 0), (1, 32768, 0),              # rows read by their own workgroup
+    (1, 32769, 4097), (3, 65536, 8192), (3, 65537, 4097), (32, 128256, 8016), (1, 2097152, 8192),
+    (1, 2097153, 0), (1, 2147483647, 0),                  # too long for groups of 256 logits
+    (0, 128256, 0), (-1, 128256, 0), (1, 0, 0), (1, -5, 0),
+])
+def test_sample_scratch_size(lib, batch, vocab, groups):
+    """4 bytes for each group of logits (4 * 2^s of them, at most 8192 groups) of each row."""
+    assert lib.mk_sample_scratch_bytes(batch, vocab) == max(batch, 0) * groups * 4
+
+
+@pytest.mark.parametrize("scratch,nbytes,code", [
+    (0x1000, 2 * 8016 * 4 - 1, -3), (0x1000, 0, -3), (0x1002, 1 << 20, -3),
+])
+def test_sample_rejects_bad_scratch(lib, scratch, nbytes, code):
+    import mk_lib
+    a = mk_lib.MkSampleArgs(0x10000, 2, 128256, 128256, 0x20000, 1, None, 0x30000, None, None)
+    assert lib.mk_sample_with_scratch(ctypes.byref(a), c_void_p(scratch), nbytes) == code
+    assert lib.mk_sample_last_error()
