@@ -137,7 +137,7 @@ struct SLds {
   uint32_t cnt[2][ST / 64];        // counts of each wave, alternating by step
   uint32_t wmin[ST / 64], wmax[ST / 64];
   uint16_t glist[MAX_GROUPS];      // the groups that hold candidates
-  uint32_t prefix, need, ncand, ngl, crowded;
+  uint32_t prefix, need, ncand, nties, ngl, crowded;
   int bin, at_bin, n, nkeep, pick;
 };
 
@@ -294,7 +294,7 @@ __device__ __forceinline__ uint32_t count_ge(const uint32_t (&v)[NG], uint32_t t
 // logits at or above the k-th largest unless more than CAND tie with it), from
 // the group maxima gm (NG per thread: groups threadIdx.x + j * ST, 0 past the
 // last; at least k groups); low and top: keys no candidate is below or above.
-// False: they do not fit, L.cand holds nothing of use.
+// False: they do not fit, L.cand holds nothing of use; at least k logits reach low.
 __device__ bool gather_top(const float* x, int V, int gs, int ngroups, int k, const uint32_t (&gm)[NG], SLds& L,
                            uint32_t& low, uint32_t& top) {
   const int t = threadIdx.x, wave = t >> 6;
@@ -384,7 +384,10 @@ __device__ bool gather_top(const float* x, int V, int gs, int ngroups, int k, co
   __syncthreads();
   gather(first, 0xffffffffu, SORT + 1u);
   __syncthreads();
-  if (L.ncand > (uint32_t)SORT) return false;
+  if (L.ncand > (uint32_t)SORT) {   // (so more than k logits reach `first`)
+    low = first;
+    return false;
+  }
   if (ties && L.ncand < (uint32_t)k) {   // the k-th largest logit is lo itself
     list_groups(L0, L0);                 // (behind the groups above lo, which may hold ties too)
     __syncthreads();
@@ -398,13 +401,16 @@ __device__ bool gather_top(const float* x, int V, int gs, int ngroups, int k, co
 
 // The same by an exact radix select over the whole row: 4 passes of 8-bit count
 // histograms over the keys find the k-th largest, then the logits above it and
-// as many ties as there is room for are gathered.
-__device__ void radix_top(const float* x, int V, int k, SLds& L) {
+// as many ties as there is room for are gathered. At least k keys reach `from`;
+// those below it are not counted (the histogram's atomics on the one or two
+// ranges that hold most of a row are what takes the time: a mask that leaves
+// 5000 logits side by side, top-k 1024: 265 -> 160 us, sorted logits 287 -> 184).
+__device__ void radix_top(const float* x, int V, int k, uint32_t from, SLds& L) {
   const int t = threadIdx.x;
   if (t == 0) {
     L.prefix = 0u;
     L.need = (uint32_t)k;
-    L.ncand = 0u;
+    L.ncand = L.nties = 0u;
   }
   uint32_t mask = 0u;
   for (int shift = 24; shift >= 0; shift -= 8) {
@@ -413,7 +419,7 @@ __device__ void radix_top(const float* x, int V, int k, SLds& L) {
     const uint32_t prefix = L.prefix;
     for (int i = t; i < V; i += ST) {
       const uint32_t kx = okey(x[i]);
-      if ((kx & mask) == prefix) atomicAdd(&L.hist[(kx >> shift) & 255u], 1u);
+      if (kx >= from && (kx & mask) == prefix) atomicAdd(&L.hist[(kx >> shift) & 255u], 1u);
     }
     __syncthreads();
     if (t == 0) {
@@ -429,18 +435,15 @@ __device__ void radix_top(const float* x, int V, int k, SLds& L) {
     mask |= 255u << shift;
     __syncthreads();
   }
-  const uint32_t thr = L.prefix;   // key of the k-th largest logit
-  for (int pass = 0; pass < 2; ++pass) {   // fewer than k above it, then the ties
-    for (int i = t; i < V; i += ST) {
-      const uint32_t kx = okey(x[i]);
-      if (pass == 0 ? kx > thr : kx == thr) {
-        const uint32_t s = atomicAdd(&L.ncand, 1u);
-        if (s < (uint32_t)CAND) L.cand[s] = ((unsigned long long)kx << 32) | (0xffffffffu - (uint32_t)i);
-      }
-    }
-    __syncthreads();
+  const uint32_t thr = L.prefix, above = (uint32_t)k - L.need;   // key of the k-th largest logit, and how many are above it
+  for (int i = t; i < V; i += ST) {
+    const uint32_t kx = okey(x[i]);
+    if (kx < thr) continue;
+    const uint32_t s = kx > thr ? atomicAdd(&L.ncand, 1u) : above + atomicAdd(&L.nties, 1u);
+    if (s < (uint32_t)CAND) L.cand[s] = ((unsigned long long)kx << 32) | (0xffffffffu - (uint32_t)i);
   }
-  if (t == 0 && L.ncand > (uint32_t)CAND) L.ncand = (uint32_t)CAND;
+  __syncthreads();
+  if (t == 0) L.ncand = above + L.nties < (uint32_t)CAND ? above + L.nties : (uint32_t)CAND;
   __syncthreads();
 }
 
@@ -586,10 +589,11 @@ __global__ void __launch_bounds__(ST) mk_sample_kernel(SParams p, const uint32_t
     if (t == 0) L.ncand = (uint32_t)V;
     __syncthreads();
   } else if (!gs || k > ngroups || !gather_top(x, V, gs, ngroups, k, gm, L, low, top)) {
+    const uint32_t from = low;   // (gather_top's, or 0)
     low = 0u;
     top = 0xffffffffu;
     __syncthreads();
-    radix_top(x, V, k, L);
+    radix_top(x, V, k, from, L);
   }
   // sorted descending (key, then ascending index); the k-th and its ties are kept
   const int nc = (int)L.ncand;

@@ -200,3 +200,46 @@ def test_sample_edges(V, pad):
             assert k != 1, (kind, int(tok[b]), ref)
             lo, hi = cdf_bracket(y, k, tp, 0.8, int(tok[b]))
             assert lo - 1e-5 <= ref_u < hi + 1e-5, (kind, k, int(tok[b]), ref, lo, hi, ref_u)
+
+
+@pytest.mark.parametrize("V,pad", [(32769, 1), (65537, 0), (262145, 3), (600001, 3), (1048577, 0), (2097152, 0), (2097153, 3)])
+def test_sample_long_rows(V, pad):
+    """Rows of every group size (8 to 256 logits, lanes of a wave that share a
+    group's maximum from 2 to 64; behind 2097152 logits none, an exact radix
+    select), with and without scratch: ordinary ones, sorted ones and ones whose
+    mask leaves one range of 5000 (both more than the search gathers: the radix
+    select over the keys that can be among the best). The oracle's tokens, or
+    ones of its CDF bracket widened by 1e-5 (fp32 sums)."""
+    need_gpu()
+    import ctypes
+    import mk_lib
+    from oracle.sampling_ref import cdf_bracket, sample
+    g = torch.Generator().manual_seed(V)
+    rows = [(kind, k) for kind in ("normal", "sorted", "range") for k in (1, 50, 0)]
+    B = len(rows)
+    store = torch.zeros(B, V + pad)
+    for b, (kind, _) in enumerate(rows):
+        x = torch.randn(V, generator=g) * 2
+        if kind == "sorted":
+            x = x.sort(descending=True).values
+        elif kind == "range":
+            x[:V - 6001] = float("-inf")
+            x[V - 1001:] = float("-inf")
+        store[b, :V] = x
+    logits = store.cuda()[:, :V]
+    params = torch.tensor([(k, 0.95, 0.8) for _, k in rows], dtype=torch.float32).cuda()
+    counter = torch.arange(B, dtype=torch.int32).cuda()
+    tok, _ = run(logits, params, 5, counter)
+    plain = torch.full((B,), -7, dtype=torch.int32, device="cuda")
+    a = mk_lib.MkSampleArgs(logits.data_ptr(), B, V, logits.stride(0), params.data_ptr(), 5, counter.data_ptr(),
+                            plain.data_ptr(), None, mk_lib.current_stream_ptr())
+    assert mk_lib.load().mk_sample(ctypes.byref(a)) == 0
+    torch.cuda.synchronize()
+    assert tok.tolist() == plain.tolist()
+    for b, (kind, k) in enumerate(rows):
+        x = store[b, :V].numpy()
+        ref, ref_u = sample(x, k, 0.95, 0.8, 5, b, b)
+        if tok[b] != ref:
+            assert k != 1, (kind, int(tok[b]), ref)
+            lo, hi = cdf_bracket(x, k, 0.95, 0.8, int(tok[b]))
+            assert lo - 1e-5 <= ref_u < hi + 1e-5, (kind, k, int(tok[b]), ref, lo, hi, ref_u)
