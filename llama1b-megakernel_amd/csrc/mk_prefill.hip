@@ -848,14 +848,15 @@ constexpr GemmTile TILES[] = {{64, 64, 2.73f, 0.50f, 0.13f},    {128, 128, 0.34f
                               {192, 128, -1.88f, 8.42f, 0.32f}, {256, 128, -0.94f, 10.66f, 0.37f},
                               {192, 128, 8.99f, -0.77f, 0.33f}, {160, 256, 0.30f, 10.96f, 0.45f},
                               {256, 256, -2.26f, 19.51f, 0.54f}};
-// The tiles each epilogue is built on: [first, end) of TILES. Those above 256x128
-// hardly ever win for N = 2048, those above 192x128 with K split; short calls are
-// the fastest on 64x64 in pairs.
+// The tiles each epilogue is built on: [first, end) of TILES. Unsplit, N = 2048
+// never takes 64x64 (K is split wherever it would) and hardly ever one above 256x128;
+// with K split those above 192x128 hardly ever win; short calls are the fastest on
+// 64x64 in pairs.
 struct TileRange {
   int first, end;
 };
 constexpr TileRange tiles_of(int epi) {
-  return epi == EPI_RES ? TileRange{0, 4} : epi == EPI_PART ? TileRange{0, 3} : epi == EPI_PAIR ? TileRange{0, 1}
+  return epi == EPI_RES ? TileRange{1, 4} : epi == EPI_PART ? TileRange{0, 3} : epi == EPI_PAIR ? TileRange{0, 1}
                                                                                                : TileRange{0, 7};
 }
 

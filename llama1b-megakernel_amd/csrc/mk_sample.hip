@@ -127,6 +127,7 @@ __host__ __device__ inline int group_size(int vocab) {
   while ((vocab + gs - 1) / gs > MAX_GROUPS) gs *= 2;
   return gs;
 }
+static_assert(SORT / 4 >= MAXK && MAX_GROUPS / 2 >= MAXK, "at least k groups, in groups of 4 and of more");
 
 struct SLds {
   uint32_t hist[BINS];             // counts of a histogram, then its start offsets
@@ -588,7 +589,7 @@ __global__ void __launch_bounds__(ST) mk_sample_kernel(SParams p, const uint32_t
     for (int i = t; i < V; i += ST) L.cand[i] = ((unsigned long long)okey(x[i]) << 32) | (0xffffffffu - (uint32_t)i);
     if (t == 0) L.ncand = (uint32_t)V;
     __syncthreads();
-  } else if (!gs || k > ngroups || !gather_top(x, V, gs, ngroups, k, gm, L, low, top)) {
+  } else if (!gs || !gather_top(x, V, gs, ngroups, k, gm, L, low, top)) {
     const uint32_t from = low;   // (gather_top's, or 0)
     low = 0u;
     top = 0xffffffffu;
