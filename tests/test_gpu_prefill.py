@@ -245,12 +245,13 @@ def test_prefill_flag_needs_batched_workspace(setup):
 
 
 @pytest.mark.timeout(300)
-@pytest.mark.parametrize("n", [200, 383, 1500])
+@pytest.mark.parametrize("n", [200, 383, 1500, 1700])
 def test_layers_prefill_matches_chunks(n):
-    """Prompts whose "layers" prefill takes each GEMM path: 200 tokens (the QKV
-    projection split over K in 4 parts, O and down in 8), 383 (QKV in 2, O and
-    down in 4), 1500 (12 row tiles of 128 tokens occupy the device: every
-    projection unsplit, the residual add in the GEMM epilogue). Their K/V rows
+    """Prompts whose "layers" prefill takes each GEMM path behind the short calls'
+    (the 70-token prompt's, whose projections are all split but gate/up): 200
+    tokens (the O projection split over K in 2 parts, down in 8), 383 (in 2 and
+    5), 1500 (O unsplit, the residual add in the GEMM epilogue, down in 2), 1700
+    (every projection unsplit). Their K/V rows
     agree with the "chunks" method's within the same relative bounds as the
     70-token prompt's against the oracle, and so does the first decode step
     from each cache (per-step bounds)."""
