@@ -481,12 +481,12 @@ struct AttnArgs {
   uint16_t* att;         // A-tile order [T16][2048]
   float* part;           // key splits: o of (split, token, q head) [64], then (max, sum) of each
   int T, p0, s_max;
-  int b0, nb;            // the launch's blocks of tokens
+  int nb;                // blocks of tokens
   int split;             // keys per split (a multiple of KB); short calls: short_split instead
   int nsplit;
 };
 // The rows a launch of pf_attn is for: any, or a short call's (early: before EARLY_ROWS).
-enum : int { ANY = 0, SHORT_EARLY = 1, SHORT_LATE = 2 };
+enum : int { ANY = 0, SHORT_EARLY = 1, SHORT_LATE = 2, SHORT_BOTH = 3 };
 
 constexpr int KB = 64;                // keys per step
 constexpr int VT_LD = KB + 8;         // bf16 per row (one dim) of the transposed V tile: 144 bytes
@@ -542,7 +542,7 @@ __global__ void __launch_bounds__(NT, NTL > 2 ? 2 : 3) pf_attn(AttnArgs a) {
   const int skew = ROWS == ANY ? 0 : a.p0 & 15;   // rows of the call's first block before its first token
   const int g = blockIdx.x & 7;                // kv head
   static_assert(NKV == 8, "a kv head per XCD");
-  const int tb = a.b0 + a.nb - 1 - ((int)blockIdx.x >> 3) % a.nb, sp = ((int)blockIdx.x >> 3) / a.nb;
+  const int tb = a.nb - 1 - ((int)blockIdx.x >> 3) % a.nb, sp = ((int)blockIdx.x >> 3) / a.nb;
   const int t0 = tb * 16 * NTL - skew;
   const int k_end = a.p0 + min(t0 + 16 * NTL, a.T);
   const int split = ROWS == ANY ? a.split : short_split(a.p0 + t0);
@@ -637,12 +637,6 @@ __global__ void __launch_bounds__(NT, NTL > 2 ? 2 : 3) pf_attn(AttnArgs a) {
     }
   };
   auto compute = [&](int k0, const AttnTile& cur) {
-    if constexpr (ROWS == SHORT_EARLY) {
-      static_assert(NTL == 1 && !SPLIT && EARLY_ROWS <= SHORT_WHOLE, "one tile, all keys");
-      compute_half(k0, 0, cur);
-      compute_half(k0, 1, cur);
-      return;
-    }
     // S^T: keys 16 kt + 4 q4 + i of the step, this lane's token of each tile
     f32x4 s[NTL][4];
 #pragma unroll
@@ -711,20 +705,34 @@ __global__ void __launch_bounds__(NT, NTL > 2 ? 2 : 3) pf_attn(AttnArgs a) {
   store_v(v[0], L[0]);
   wait_copies<FLY, 0>();
   const int steps = (n_keys - key0 + KB - 1) / KB;
-  int slot = 0;
-  for (int it = 0; it < steps; it += 2) {
+  auto run_steps = [&](auto early) {
+    int slot = 0;
+    for (int it = 0; it < steps; it += 2) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      if (it + u < steps) {
-        const int k0 = key0 + (it + u) * KB, s1 = slot == ANS - 1 ? 0 : slot + 1, s2 = s1 == ANS - 1 ? 0 : s1 + 1;
-        load_v(k0 + 2 * KB, v[u]);
-        stage_k(k0 + 2 * KB, L[s2]);
-        compute(k0, L[slot]);
-        store_v(v[u ^ 1], L[s1]);
-        wait_copies<FLY, 0>();
-        slot = s1;
+      for (int u = 0; u < 2; ++u) {
+        if (it + u < steps) {
+          const int k0 = key0 + (it + u) * KB, s1 = slot == ANS - 1 ? 0 : slot + 1, s2 = s1 == ANS - 1 ? 0 : s1 + 1;
+          load_v(k0 + 2 * KB, v[u]);
+          stage_k(k0 + 2 * KB, L[s2]);
+          if constexpr (early.value) {
+            static_assert(NTL == 1 && !SPLIT && EARLY_ROWS <= SHORT_WHOLE, "one tile, all keys");
+            compute_half(k0, 0, L[slot]);
+            compute_half(k0, 1, L[slot]);
+          } else {
+            compute(k0, L[slot]);
+          }
+          store_v(v[u ^ 1], L[s1]);
+          wait_copies<FLY, 0>();
+          slot = s1;
+        }
       }
     }
+  };
+  if constexpr (ROWS == SHORT_BOTH) {
+    if (a.p0 + t0 < EARLY_ROWS) run_steps(std::true_type{});
+    else run_steps(std::false_type{});
+  } else {
+    run_steps(std::bool_constant<ROWS == SHORT_EARLY>{});
   }
   // the token's sum over its four lanes; o = acc / l, dims 16 d + 4 q4 + i
 #pragma unroll
@@ -793,23 +801,18 @@ void attn_launch(const AttnArgs& a, hipStream_t st) {
 // (33 tokens at 4000 rows: 55 us whole, 17.5 in 8 parts; at 700 rows 13.6 and
 // 11.0). Splits begin at multiples of 64 keys of the cache.
 //
-// Short calls split a token's keys by its row alone (short_split); a call across
-// EARLY_ROWS takes a launch for the rows on either side (no keys are split there).
+// Short calls split a token's keys by its row alone (short_split). One across
+// EARLY_ROWS takes a kernel with both forms of a step: 33 tokens at row 100 49.7 us,
+// with a launch for either side 54.9. The other calls would lose 0.7 us by it.
 void attn_run(AttnArgs a, hipStream_t st) {
-  a.b0 = 0;
   if (a.T <= SHORT_TOKENS) {
-    const int base = a.p0 & ~15, nb = (a.p0 + a.T - base + 15) / 16;
-    const int early = min(max((EARLY_ROWS - base) / 16, 0), nb);
+    const int base = a.p0 & ~15;
+    a.nb = (a.p0 + a.T - base + 15) / 16;
     a.nsplit = 1;
     for (int row = base; row < a.p0 + a.T; row += 16)
       a.nsplit = max(a.nsplit, (min(row + 16, a.p0 + a.T) + short_split(row) - 1) / short_split(row));
-    if (early) {
-      a.nb = early;
-      attn_launch<1, false, SHORT_EARLY>(a, st);
-    }
-    a.b0 = early;
-    a.nb = nb - early;
-    if (!a.nb) return;
+    if (a.p0 + a.T <= EARLY_ROWS) return attn_launch<1, false, SHORT_EARLY>(a, st);
+    if (a.p0 < EARLY_ROWS) return attn_launch<1, false, SHORT_BOTH>(a, st);
     if (a.nsplit == 1) return attn_launch<1, false, SHORT_LATE>(a, st);
     return attn_launch<1, true, SHORT_LATE>(a, st);
   }
