@@ -1546,9 +1546,9 @@ __device__ __forceinline__ void phase_lm(BCtx& c, BLds<MT>& L, uint32_t epoch) {
 // GFIX: the grid size when known at compile time (the per-phase work splits
 // then divide by a constant); 0: gridDim.x.
 // ONE: a step of exactly one layer. Without the layer loop nothing is hoisted
-// in front of it: those 1400 instructions between the first QKV phase and its
-// attention (which the loop's later layers gain from) took a one-layer launch
-// 3 us. Batch 3: 38.8 -> 36.9 us; batch 20 behind up to 4000 rows: 63.2 -> 62.4.
+// in front of it: 1400 instructions between the first QKV phase and its attention
+// (which the loop's later layers gain from). Batch 3: 38.8 -> 36.9 us; batch 20
+// behind up to 4000 rows: 63.2 -> 62.4.
 template <int MT, int GFIX, bool ONE>
 __global__ void __launch_bounds__(NT, 1) mk_batch_kernel(BParams p) {
   __shared__ BLds<MT> L;

@@ -101,8 +101,8 @@ __device__ __forceinline__ void wait_copies() {
 // each at one wave per SIMD and got 770-850 TFLOP/s; 256x256 on eight waves of
 // 128x64 halves the copies per MFMA and puts two waves on a SIMD, so that one
 // multiplies while the other waits: 16384 x 2048 weights at 3000 tokens 208 ->
-// 147 us (1370 TFLOP/s). Smaller tiles serve the shapes that would leave the
-// device idle (gemm_tile).
+// 147 us timed alone (1370 TFLOP/s; 163 in a layer). Smaller tiles serve the shapes
+// that would leave the device idle (gemm_tile).
 //
 // Operands are 1 KiB blocks (16 rows x 32 columns) copied from memory straight
 // into a ring of NS k-steps in LDS, NS - 1 ahead; each wave reads the next
