@@ -886,9 +886,10 @@ void gemm_run(GemmArgs g, int tile, hipStream_t st) {
 }
 
 // The estimated time of a projection of M tokens. A split adds what it moves (its
-// partials' bytes at 7 TB/s: a weight that chooses well, not a bandwidth, since the
-// fitted times hold the GEMM's own stores) less 0.5 us, as its tail takes the place
-// of pf_norm.
+// partials' bytes at 7 TB/s: a weight, not a bandwidth, since the fitted times hold
+// the GEMM's own stores) less 0.5 us, as its tail takes the place of pf_norm. Four
+// times that weight chooses fewer parts: a layer of 200 tokens then takes 72 us
+// instead of 69, one of 512 102.6 instead of 104.3, of 900 157 instead of 156.
 float gemm_us(const GemmTile& t, int M, int N, int K, int splits) {
   const int wg = (M + t.tm - 1) / t.tm * (N / t.tn) * splits;
   const float rounds = t.tm == 64 ? fmaxf(1.f, (float)wg / 256.f) : (float)((wg + 255) / 256);
