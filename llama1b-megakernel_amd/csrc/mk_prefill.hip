@@ -930,6 +930,9 @@ int gemm_splits(int M, int N, int K, size_t part_bytes) {
 // time (5, 8 and 8), 128 tokens at row 200: 61 us; every part stored and every
 // maximum over 32 keys there: 55 and 71 us.
 constexpr int SHORT_QKV = 8, SHORT_RES = 16;
+static_assert((size_t)SHORT_TOKENS * 4 * SHORT_QKV * QKV_ROWS <= PART_BYTES &&
+                  (size_t)SHORT_TOKENS * 4 * SHORT_RES * H <= PART_BYTES,
+              "a short call's partials fit");
 void gemm_short(GemmArgs g, int parts, hipStream_t st) {
   const bool pairs = g.p0 >= EARLY_ROWS;
   g.splits = pairs ? parts / 2 : parts;
